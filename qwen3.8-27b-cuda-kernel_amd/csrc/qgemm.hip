@@ -10,15 +10,15 @@
 //   * v_mfma_f32_32x32x16_bf16 with the activations as the A operand and the weights as B. A lane
 //     of the B operand holds eight consecutive k of one column; the repacked weights
 //     (bq_repack.cpp) give it those codes as one 16-byte word per 64-k group (+ the high bits).
-//   * The codes enter the MFMA as the exact bf16 values 128 + u (u = the stored unsigned code, two
-//     bit operations per pair), so no conversion arithmetic is spent on them; the offset and the
-//     per-(column, group) scale are applied once per group in fp32:
+//   * Up to 32 rows the codes enter the MFMA as the exact bf16 values 128 + u (u = the stored unsigned
+//     code, two bit operations per pair), so no conversion arithmetic is spent on them; the offset and
+//     the per-(column, group) scale are applied once per group in fp32:
 //       C += scale[n][g] * (T_g - (128 + 2^(b-1)) * S_g),  T_g = sum_{k in g} a[m][k] (128 + u),
 //     where S_g = sum_{k in g} a[m][k] comes from one more MFMA against a ones operand (its output
 //     lands in the same registers as T's rows). T carries at most ~8 bits of cancellation; the
-//     result keeps ~16 significant bits, far below the bf16 output's rounding.
-//   * A workgroup is four waves over a 32 MB-row x 256-column tile (a wave: 64 columns, two MFMA
-//     column blocks); the K loop walks 64-wide groups with the next group's loads in flight.
+//     result keeps ~16 significant bits, far below the bf16 output's rounding. With more rows a
+//     workgroup dequantises its columns once into LDS, for up to 1,024 rows or so as the exact signed
+//     codes (the scale still in fp32, once per group), beyond as bf16(code x scale).
 //   * Small M leaves too few tiles to pull the weights at HBM speed, so K is split over several
 //     workgroups: each writes its fp32 partial tile (rows < M only) with write-through stores,
 //     counts its arrival on a per-tile counter, and the last to arrive sums the slices in slice
@@ -41,21 +41,19 @@ int launch_qk_norm_rope_append(const q38a_qk_norm_rope_params& p, const q38a_bat
 
 namespace {
 
-// A workgroup covers 256 columns: 8 waves of one 32-column block for one row block (small M: more
-// waves, each with fewer registers, keep more weight bytes in flight), 4 waves of two blocks for two
-// row blocks (more reuse of each A operand).
+// A workgroup of the small-M kernel covers 32 rows x 256 columns: two sets (K parts) of 8 waves of
+// one 32-column block, each set over half the slice's groups (twice the weight bytes in flight per
+// CU), their sums added through LDS.
 constexpr int kTileN = 256;
-constexpr int kMaxWaves = 8;
-__host__ __device__ constexpr int nb_of(int mb) { return mb == 1 ? 1 : 2; }      // 32-column blocks per wave
-__host__ __device__ constexpr int waves_of(int mb) { return kTileN / (32 * nb_of(mb)); }
-// K parts of a workgroup's slice: one row block runs two sets of 8 waves, each over half the slice's
-// groups (twice the weight bytes in flight per CU), their sums added through LDS
-__host__ __device__ constexpr int kparts_of(int mb) { return mb == 1 ? 2 : 1; }
-__host__ __device__ constexpr int threads_of(int mb) { return 64 * waves_of(mb) * kparts_of(mb); }
+constexpr int kColWaves = kTileN / 32;
+constexpr int kKParts = 2;
+constexpr int kGemvThreads = 64 * kColWaves * kKParts;
 constexpr int kEpiFused = 100;  // epilogue kind of the fused in-projection
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
 
 struct GemmArgs {
   const uint16_t* a;
@@ -73,6 +71,7 @@ struct GemmArgs {
   int norm_blocks;
   float inv_hidden, eps;
   int tiles_n, splits;
+  int wide_out;  // the epilogue's buffers take 16-byte accesses (alignment of pointers and row strides)
   float* ws_partials;
   int* counters;
 };
@@ -186,44 +185,37 @@ __device__ inline float row_scale(const GemmArgs& a, int row) {
 
 struct alignas(16) GemmShared {
   union {
-    uint16_t tile[64][kTileN + 8];  // fused epilogue: the bf16 head tile (rows x 256)
-    float resid_ss[kMaxWaves][64];  // residual epilogue: per-wave sums of squares of its columns
-    float kpart[kMaxWaves][16][64];  // the second K part's sums (one row block, one column block)
+    uint16_t tile[32][kTileN + 8];   // fused epilogue: the bf16 head tile (rows x 256)
+    float resid_ss[kColWaves][32];   // residual epilogue: per-wave sums of squares of its columns
+    float kpart[kColWaves][16][64];  // the second K part's sums
   };
-  double stage[kMaxWaves][kHeadDim];  // the append's sequential-sum fallback
-  float rs[64];                       // row scales of the folded RMSNorm (1 without partials_in)
+  double stage[kColWaves][kHeadDim];  // the append's sequential-sum fallback
+  float rs[32];                       // row scales of the folded RMSNorm (1 without partials_in)
   int last;
 };
 
-// The tile's end, shared by both kernels: split-K slices summed by the last workgroup to arrive,
-// then the epilogue. C element e of (row block mb, column block j) in this lane: row
-// 32 mb + 8 (e / 4) + 4 (lane / 32) + e % 4 of the tile, column 32 (kNB wave + j) + lane % 32. Every
-// wave of the column tile calls it (K-part waves have ended); sh.rs holds the tile's row scales.
+// The small-M kernel's end: split-K slices summed by the last workgroup to arrive, then the epilogue.
+// C element e in this lane: row 8 (e / 4) + 4 (lane / 32) + e % 4, column 32 wave + lane % 32 of the
+// tile. Every wave of the column tile calls it (K-part waves have ended); sh.rs holds the rows' scales.
 // EQ: row quads of the MFMA output that can hold rows < M (the split-K traffic skips the others).
-template <int MB, bool FUSED, int EQ = 4>
+template <bool FUSED, int EQ>
 __device__ void tile_finish(const GemmArgs& a, const AppendArgs& ap, const BatchArgs& batch, const KvArgs& kv,
-                            GemmShared& sh, float16_t (&C)[MB][nb_of(MB)], int tile, int z, int tn, int wave,
-                            int lane) {
-  constexpr int kNB = nb_of(MB), kGWaves = waves_of(MB), kBM = 32 * MB;
+                            GemmShared& sh, float16_t& C, int tn, int z, int wave, int lane) {
+  constexpr int kRows = 32;
   const int kg = lane >> 5;
-  const int m0 = (tile / a.tiles_n) * kBM;
-  auto row_of = [&](int mb, int e) { return m0 + 32 * mb + 8 * (e >> 2) + 4 * kg + (e & 3); };
-  const int colw = tn * kTileN + 32 * kNB * wave + (lane & 31);  // + 32 j
+  auto row_of = [&](int e) { return 8 * (e >> 2) + 4 * kg + (e & 3); };
+  const int col = tn * kTileN + 32 * wave + (lane & 31);
 
   // ---- split-K: the last of the tile's slices sums them in slice order -------------------------
   if (a.splits > 1) {
-    float* part = a.ws_partials + size_t(tile) * a.splits * kBM * kTileN;
+    float* part = a.ws_partials + size_t(tn) * a.splits * kRows * kTileN;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int j = 0; j < kNB; ++j)
-#pragma unroll
-        for (int e = 0; e < 4 * EQ; ++e) {
-          const int r = row_of(mb, e) - m0;
-          if (m0 + r < a.m)
-            __hip_atomic_store(part + (size_t(z) * kBM + r) * kTileN + 32 * (kNB * wave + j) + (lane & 31), C[mb][j][e],
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+    for (int e = 0; e < 4 * EQ; ++e) {
+      const int r = row_of(e);
+      if (r < a.m)
+        __hip_atomic_store(part + (size_t(z) * kRows + r) * kTileN + 32 * wave + (lane & 31), C[e], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
     // Hand-off without release/acquire fences: the partials are agent-scope atomic stores, which
     // gfx950 issues write-through past the XCD's L2 (sc1), s_waitcnt(0) waits until every one has
     // completed, the barrier orders all threads' completed stores before thread 0's arrival count,
@@ -234,9 +226,9 @@ __device__ void tile_finish(const GemmArgs& a, const AppendArgs& ap, const Batch
     __builtin_amdgcn_s_waitcnt(0);  // the write-through stores have completed
     __syncthreads();
     if (threadIdx.x == 0) {
-      const int old = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int old = __hip_atomic_fetch_add(a.counters + tn, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       sh.last = old == a.splits - 1;
-      if (sh.last) __hip_atomic_store(a.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (sh.last) __hip_atomic_store(a.counters + tn, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
     if (!sh.last) return;
@@ -244,288 +236,610 @@ __device__ void tile_finish(const GemmArgs& a, const AppendArgs& ap, const Batch
     // with agent-coherent (sc1) buffer loads; kZB slices' loads are issued together (a batch past
     // the last slice re-reads the last one and discards it)
     const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
-        part, short(0), int(size_t(a.splits) * kBM * kTileN * sizeof(float)), 0x00020000);
+        part, short(0), int(size_t(a.splits) * kRows * kTileN * sizeof(float)), 0x00020000);
     constexpr int kSc1 = 16;  // cache policy bit sc1
-    constexpr int kZB = MB == 1 ? 16 / EQ : 2;
+    constexpr int kZB = 16 / EQ;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int j = 0; j < kNB; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) C[mb][j][e] = 0.0f;
+    for (int e = 0; e < 16; ++e) C[e] = 0.0f;
     for (int zb = 0; zb < a.splits; zb += kZB) {
-      float V[kZB][MB][kNB][4 * EQ];
+      float V[kZB][4 * EQ];
 #pragma unroll
       for (int q = 0; q < kZB; ++q) {
         const int zz = zb + q < a.splits ? zb + q : a.splits - 1;
-        const int zoff = zz * kBM * kTileN * int(sizeof(float));
+        const int zoff = zz * kRows * kTileN * int(sizeof(float));
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-          for (int j = 0; j < kNB; ++j)
-#pragma unroll
-            for (int e = 0; e < 4 * EQ; ++e) {
-              const int r = row_of(mb, e) - m0;
-              const int off = (r * kTileN + 32 * (kNB * wave + j) + (lane & 31)) * int(sizeof(float));
-              V[q][mb][j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(prs, off, zoff, kSc1));
-            }
+        for (int e = 0; e < 4 * EQ; ++e) {
+          const int off = (row_of(e) * kTileN + 32 * wave + (lane & 31)) * int(sizeof(float));
+          V[q][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(prs, off, zoff, kSc1));
+        }
       }
 #pragma unroll
       for (int q = 0; q < kZB; ++q) {
         const bool use = zb + q < a.splits;
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-          for (int j = 0; j < kNB; ++j)
-#pragma unroll
-            for (int e = 0; e < 4 * EQ; ++e) C[mb][j][e] = use ? C[mb][j][e] + V[q][mb][j][e] : C[mb][j][e];
+        for (int e = 0; e < 4 * EQ; ++e) C[e] = use ? C[e] + V[q][e] : C[e];
       }
     }
   }
 
   // ---- epilogues --------------------------------------------------------------------------------
   if (a.splits == 1) __syncthreads();  // sh.rs (the split-K path has passed barriers already)
+  float rs[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) rs[e] = sh.rs[row_of(e)];
   if constexpr (FUSED) {
     const int head = tn;  // proj column blocks: q heads, gate heads, k heads, v heads
     const int nq = ap.nq, nkv = ap.nkv;
     const bool is_gate = head >= nq && head < 2 * nq;
-    float rs[MB][4][4];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) rs[mb][i][r] = sh.rs[row_of(mb, 4 * i + r) - m0];
     if (is_gate) {
       uint16_t* out = static_cast<uint16_t*>(a.out);
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int j = 0; j < kNB; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const int row = row_of(mb, e);
-            if (row < a.m) out[size_t(row) * a.ldo + colw + 32 * j] = bf16_bits(C[mb][j][e] * rs[mb][e >> 2][e & 3]);
-          }
+      for (int e = 0; e < 16; ++e) {
+        const int row = row_of(e);
+        if (row < a.m) out[size_t(row) * a.ldo + col] = bf16_bits(C[e] * rs[e]);
+      }
       return;
     }
     // q / k / v head: the bf16 tile (exactly what proj would hold) into LDS, then the append rows
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int j = 0; j < kNB; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          sh.tile[row_of(mb, e) - m0][32 * (kNB * wave + j) + (lane & 31)] = bf16_bits(C[mb][j][e] * rs[mb][e >> 2][e & 3]);
+    for (int e = 0; e < 16; ++e) sh.tile[row_of(e)][32 * wave + (lane & 31)] = bf16_bits(C[e] * rs[e]);
     __syncthreads();
     const int rtype = head < nq ? head : (head < 2 * nq + nkv ? nq + (head - 2 * nq) : nq + nkv + (head - 2 * nq - nkv));
-    for (int r = wave; r < kBM && m0 + r < a.m; r += kGWaves) {
+    for (int r = wave; r < kRows && r < a.m; r += kColWaves) {
       RowLoads L;
-      L.m = m0 + r;
+      L.m = r;
       L.r = rtype;
       L.pos = batch.tok_pos[L.m];
       L.raw = *reinterpret_cast<const uint2*>(&sh.tile[r][4 * lane]);
       row_meta(ap, batch, kv, lane, L);
       append_row(ap, kv, sh.stage[wave], lane, L);
     }
-    return;
-  } else {
-    if (a.kind == Q38A_EPI_RESIDUAL) {
-      // residual += C; xbf = bf16(residual); sums of squares per 128 columns (reference
-      // qgemm.cu:356-380; the sum's order differs: per column pair of waves)
-      float ss[MB][4][4];
+  } else if (a.kind == Q38A_EPI_RESIDUAL) {
+    // residual += C; xbf = bf16(residual); sums of squares per 128 columns (reference
+    // qgemm.cu:356-380; the sum's order differs): the 32 lanes of each half wave, then the four
+    // waves of each 128-column block in wave order
+    float ss[16];
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) ss[mb][i][r] = 0.f;
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int j = 0; j < kNB; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const int row = row_of(mb, e), col = colw + 32 * j;
-            if (row < a.m) {
-              float* res = a.residual + size_t(row) * a.n + col;
-              const float x = *res + C[mb][j][e];
-              *res = x;
-              a.xbf[size_t(row) * a.n + col] = bf16_bits(x);
-              ss[mb][e >> 2][e & 3] += x * x;
-            }
-          }
-      // 32 kNB columns of this wave per row: reduce over the 32 lanes of each half, then the waves
-      // of each 128-column block in wave order
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float v = ss[mb][i][r];
-#pragma unroll
-            for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-            ss[mb][i][r] = v;
-          }
-      for (int mb = 0; mb < MB; ++mb) {
-        __syncthreads();
-        if ((lane & 31) == 0) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sh.resid_ss[wave][8 * i + 4 * kg + r] = ss[mb][i][r];
-        }
-        __syncthreads();
-        // 128-column block b: waves b wpb .. b wpb + wpb - 1
-        constexpr int wpb = 4 / kNB;
-        if (threadIdx.x < 2 * 32) {
-          const int bw = threadIdx.x >> 5, r = threadIdx.x & 31;
-          const int row = m0 + 32 * mb + r;
-          float v = 0.0f;
-#pragma unroll
-          for (int w = 0; w < wpb; ++w) v += sh.resid_ss[wpb * bw + w][r];
-          if (row < a.m) a.partials_out[size_t(row) * a.norm_blocks + (tn * kTileN) / 128 + bw] = v;
-        }
+    for (int e = 0; e < 16; ++e) {
+      const int row = row_of(e);
+      ss[e] = 0.f;
+      if (row < a.m) {
+        float* res = a.residual + size_t(row) * a.n + col;
+        const float x = *res + C[e];
+        *res = x;
+        a.xbf[size_t(row) * a.n + col] = bf16_bits(x);
+        ss[e] = x * x;
       }
-      return;
+#pragma unroll
+      for (int off = 16; off > 0; off >>= 1) ss[e] += __shfl_xor(ss[e], off, 64);
     }
-    float rs[MB][4][4];
+    __syncthreads();
+    if ((lane & 31) == 0) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+      for (int e = 0; e < 16; ++e) sh.resid_ss[wave][row_of(e)] = ss[e];
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 * kRows) {
+      const int bw = threadIdx.x >> 5, r = threadIdx.x & 31;
+      float v = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int w = 0; w < 4; ++w) v += sh.resid_ss[4 * bw + w][r];
+      if (r < a.m) a.partials_out[size_t(r) * a.norm_blocks + (tn * kTileN) / 128 + bw] = v;
+    }
+  } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) rs[mb][i][r] = sh.rs[row_of(mb, 4 * i + r) - m0];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int j = 0; j < kNB; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int row = row_of(mb, e), col = colw + 32 * j;
-          if (row >= a.m || col >= a.n_store) continue;
-          const float y = C[mb][j][e] * rs[mb][e >> 2][e & 3];
-          if (a.kind == Q38A_EPI_STORE_F32) static_cast<float*>(a.out)[size_t(row) * a.ldo + col] = y;
-          else static_cast<uint16_t*>(a.out)[size_t(row) * a.ldo + col] = bf16_bits(y);
-        }
+    for (int e = 0; e < 16; ++e) {
+      const int row = row_of(e);
+      if (row >= a.m || col >= a.n_store) continue;
+      const float y = C[e] * rs[e];
+      if (a.kind == Q38A_EPI_STORE_F32) static_cast<float*>(a.out)[size_t(row) * a.ldo + col] = y;
+      else static_cast<uint16_t*>(a.out)[size_t(row) * a.ldo + col] = bf16_bits(y);
+    }
   }
 }
 
-// Group compute shared by both kernels: T = A . (128 + u) over the group's four 16-k steps of one
-// column block, with A's steps in registers.
-template <int BITS, int MB>
-__device__ inline void group_products(float16_t (&T)[MB], const u32x4 (&Ab)[MB][4], const BWords& bw,
-                                      uint32_t magic) {
+// T = A . (128 + u) over a group's four 16-k steps of one column block, with A's steps in registers.
+template <int BITS>
+__device__ inline float16_t group_products(const u32x4 (&Ab)[4], const BWords& bw, uint32_t magic) {
+  float16_t T = float16_t{};
   auto t_step = [&](auto step) {
     constexpr int s = decltype(step)::value;
-    const bf16x8_t bo = b_operand<BITS, s>(bw, magic);
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-      T[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, Ab[mb][s]), bo,
-                                                      s == 0 ? float16_t{} : T[mb], 0, 0, 0);
+    T = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, Ab[s]), b_operand<BITS, s>(bw, magic), T, 0,
+                                                0, 0);
   };
   t_step(std::integral_constant<int, 0>{});
   t_step(std::integral_constant<int, 1>{});
   t_step(std::integral_constant<int, 2>{});
   t_step(std::integral_constant<int, 3>{});
+  return T;
 }
 
-// ---- larger M: 64 x 256 tiles, four waves of 64 x 64 ------------------------------------------
-// A and B stream from global memory, two groups in flight per wave; S_g (the rows' sums over a
-// group) from one more MFMA per step against a ones operand.
-template <int BITS, bool FUSED>
-__global__ void __launch_bounds__(threads_of(2)) __attribute__((amdgpu_waves_per_eu(2)))
-qgemm_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn) {
-  constexpr int MB = 2, kNB = nb_of(MB), kBM = 32 * MB;
-  __shared__ GemmShared sh;
+// ---- 33 rows and more: 256 x 128 or 128 x 128 tiles, exact codes -------------------------------
+// Eight waves of 64 x 64. The tile's columns are dequantised once per workgroup into LDS as the
+// exact signed codes in bf16 (MFMA B operand layout: block, step, lane, 8 k) and shared by the
+// waves of its rows; A rows come by the DMA path of buffer loads, 16-byte chunk c of a row in
+// slot c ^ (row / 2 % 8): the 16 rows that one clock of an operand read takes then fall in 16 different
+// quads of the 64 banks. Each 64-k group's products accumulate in their own registers (T, starting from
+// zero) and C += scale * T in fp32 when the group is done: the codes are exact, so the only
+// roundings are the fp32 sums'. One column block's T is folded while the other block's MFMAs run,
+// and the last one's at the start of the next step, under the latency of that step's first operand
+// reads. KP: 64-k groups per step. With 256 rows a step is one group; with 128 rows two sets of four
+// waves take one group each (the same 512 dequantised codes per step and thread, the same LDS),
+// and the sets' sums are added through LDS at the end (set 0 + set 1).
+//
+// Bound: per 64 x 64 x 64 wave step 512 MFMA cycles against 64 folds + 56 (5-bit, 256 rows) or 112
+// dequantisation instructions of 4 cycles each, i.e. the VALU, which two waves per SIMD overlap with
+// the MFMA pipe.
+constexpr int kTileWaves = 8;
+constexpr int kTileThreads = 64 * kTileWaves;
+constexpr int kTileCols = 128;  // two waves wide
+constexpr int kTileMaxSplits = 8;
+// rows per tile for WM waves of 64 rows; 64-k groups per step
+__host__ __device__ constexpr int tile_rows(int wm) { return 64 * wm; }
+__host__ __device__ constexpr int tile_kparts(int wm) { return kTileWaves / (2 * wm); }
+
+template <int WM>
+struct alignas(16) TileShared {
+  union {
+    struct {
+      u32x4 a[3][256][8];  // [buffer][group of the step, row][slot]: 256 = rows x groups for every WM
+      uint16_t b[2][tile_kparts(WM)][4][4][64][8];  // [buffer][group][block][step][lane][k]
+    } s;
+    struct {  // after the K loop
+      union {
+        float red[4][64][64];               // the second K part's sums: [wave][element][lane]
+        float out[kTileWaves][32][64 + 4];  // 32 rows of a wave's tile
+      };
+      float rs[tile_rows(WM)];     // row scales of the folded RMSNorm
+      float ss[2][tile_rows(WM)];  // residual epilogue: each wave column's sums of squares
+      int last;
+    } e;
+  };
+};
+
+// 16 bytes per lane from the buffer to LDS at dst (wave-uniform) + 16 x lane, without registers.
+__device__ inline void copy_to_lds(__amdgpu_buffer_rsrc_t r, u32x4* dst, int voffset, int soffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voffset, soffset, 0, 0);
+}
+
+// One thread's share of a step's weights: NS 16-k steps of one lane word (their low nibbles, 32
+// bits a step) and the high bits of those steps.
+template <int NS>
+struct TileWords {
+  uint32_t lo[NS];
+  u32x2 hi;
+};
+
+// Steps [first, first + NS) of lane word l of block nb, group g (nb and g wave-uniform).
+template <int BITS, int NS>
+__device__ inline void load_tile_words(TileWords<NS>& w, const BPlanes& p, int nb, int g, int G, int l, int first) {
+  const int unit = nb * G + g;
+  if constexpr (NS == 4) {
+    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(p.lo, l * 16, unit * 1024, 0));
+    w.lo[0] = v.x;
+    w.lo[1] = v.y;
+    w.lo[2] = v.z;
+    w.lo[3] = v.w;
+  } else {
+    const u32x2 v =
+        __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(p.lo, l * 16 + 4 * first, unit * 1024, 0));
+    w.lo[0] = v.x;
+    w.lo[1] = v.y;
+  }
+  if constexpr (BITS == 5) w.hi = u32x2{__builtin_amdgcn_raw_buffer_load_b32(p.hi, l * 4, unit * 256, 0), 0u};
+  else if constexpr (BITS == 6 && NS == 4)
+    w.hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(p.hi, l * 8, unit * 512, 0));
+  else if constexpr (BITS == 6)  // steps 0-1 are in the first word, 2-3 in the second
+    w.hi = u32x2{__builtin_amdgcn_raw_buffer_load_b32(p.hi, l * 8 + 2 * first, unit * 512, 0), 0u};
+  else w.hi = u32x2{0u, 0u};
+}
+
+// (x & mask) | c in one instruction (the compiler splits it over a literal AND and an OR3). Only for
+// values that vector instructions read: see and_or.
+__device__ inline uint32_t and_or_valu(uint32_t x, uint32_t mask, uint32_t c) {
+  uint32_t d;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(d) : "v"(x), "s"(mask), "v"(c));
+  return d;
+}
+
+// Codes 2P and 2P + 1 of a lane word's step as a pair of signed codes in bf16, exact. lo: the step's
+// nibbles, for P >= 2 already shifted right by 8; hi: the high bits. The fp16 values 2048 + 2 u (P
+// even) or 2048 + 32 u (P odd: the nibble stays where it is), then one mixed-precision fma per code,
+// which reads the fp16 half and takes the factor and the offset off, and one conversion of both.
+template <int BITS, int S, int P>
+__device__ inline uint32_t code_pair_bf16(uint32_t lo, uint32_t hi, uint32_t magic) {
+  constexpr int q = 4 * S + P, up = P & 1 ? 4 : 0;  // the code's lowest bit in the fp16 mantissa
+  uint32_t w = and_or_valu(lo, 0x000F000Fu << up, magic);
+  if constexpr (BITS == 5) w = and_or_valu(shr<q - 4 - up>(hi), 0x00100010u << up, w);
+  if constexpr (BITS == 6) w = and_or_valu(shr<2 * (q & 7) - 4 - up>(hi), 0x00300030u << up, w);
+  constexpr float f = P & 1 ? 1.0f / 32 : 0.5f, off = -(2048.0f * f + float(1 << (BITS - 1)));
+  const half2_t h = __builtin_bit_cast(half2_t, w);
+  const float2_t x{__builtin_fmaf(float(h.x), f, off), __builtin_fmaf(float(h.y), f, off)};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2_t));
+}
+
+// Step S of the thread's words into LDS.
+template <int BITS, int NS, int S>
+__device__ inline void tile_dequant_step(uint16_t* dst, const TileWords<NS>& w, uint32_t hi, uint32_t magic) {
+  const uint32_t lo = w.lo[S], lo8 = lo >> 8;
+  const u32x4 v{code_pair_bf16<BITS, S, 0>(lo, hi, magic), code_pair_bf16<BITS, S, 1>(lo, hi, magic),
+                code_pair_bf16<BITS, S, 2>(lo8, hi, magic), code_pair_bf16<BITS, S, 3>(lo8, hi, magic)};
+  *reinterpret_cast<u32x4*>(dst) = v;
+}
+
+template <int BITS, int WM>
+__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) qgemm_tile_kernel(GemmArgs a) {
+  constexpr int KP = tile_kparts(WM), BM = tile_rows(WM);
+  constexpr int NS = KP == 1 ? 2 : 4;  // 16-k steps each thread dequantises per step
+  __shared__ TileShared<WM> sh;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, kg = lane >> 5;
-  const int z = blockIdx.x % a.splits, tile = blockIdx.x / a.splits;
-  const int tn = tile % a.tiles_n, m0 = (tile / a.tiles_n) * kBM;
+  const int kp = wave / (2 * WM), wi = wave % (2 * WM), wm = wi >> 1, wn = wi & 1;
+  // tiles of one column block (the same weights) and its K slices on one XCD (blockIdx mod 8), when
+  // the column blocks divide evenly
+  const int tiles_m = (a.m + BM - 1) / BM, inner = tiles_m * a.splits;
+  int tn, rest;
+  if (a.tiles_n % 8 == 0) {
+    const int idx = blockIdx.x >> 3;
+    tn = (idx / inner) * 8 + (blockIdx.x & 7);
+    rest = idx % inner;
+  } else {
+    tn = blockIdx.x / inner;
+    rest = blockIdx.x % inner;
+  }
+  tn = __builtin_amdgcn_readfirstlane(tn);
+  const int tm = __builtin_amdgcn_readfirstlane(rest / a.splits), z = __builtin_amdgcn_readfirstlane(rest % a.splits);
+  const int m0 = tm * BM;
   const int G = a.k / 64;
   const int g0 = int((long long)z * G / a.splits), g1 = int((long long)(z + 1) * G / a.splits);
-  const int nb0 = tn * (kTileN / 32) + wave * kNB;  // this wave's first 32-column block
-
-  // A rows of this lane through a buffer resource over the tile's valid rows: rows past M fall
-  // outside its range and load as zero without a memory request
-  const int valid_rows = a.m - m0 < kBM ? a.m - m0 : kBM;
+  const int steps = (g1 - g0 + KP - 1) / KP;
+  const BPlanes bp = make_bplanes<BITS>(a);
+  const int valid_rows = a.m - m0 < BM ? a.m - m0 : BM;
   const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(
       uniform_ptr(const_cast<uint16_t*>(a.a) + size_t(m0) * a.k), short(0), valid_rows * a.k * int(sizeof(uint16_t)),
       0x00020000);
-  const BPlanes bp = make_bplanes<BITS>(a);
-  int aoff[MB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) aoff[mb] = ((32 * mb + (lane & 31)) * a.k + 8 * kg) * int(sizeof(uint16_t));
-  float16_t C[MB][kNB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int j = 0; j < kNB; ++j) C[mb][j] = float16_t{};
-  const float c0 = 128.0f + float(1 << (BITS - 1));
-  const uint32_t magic = 0x43004300u;  // bf16 128 in both halves
-  bf16x8_t ones;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ones[i] = __bf16(1.0f);
+  const uint32_t magic = 0x68006800u;  // fp16 2048 in both halves
 
-  // two register buffers rotate over the groups; the rotation loop is unrolled, so every buffer
-  // index is a constant
-  constexpr int kDepth = 2;
-  u32x4 A[kDepth][MB][4];
-  BWords B[kDepth][kNB];
-  auto load_group = [&](u32x4 (&Ab)[MB][4], BWords (&Bb)[kNB], int g) {
+  // the thread's lane word of the step's weights: group dkp of the step, block db, lane dl; with one
+  // group per step, steps 2 dh and 2 dh + 1 of it
+  const int dkp = KP == 1 ? 0 : wave >> 2, db = wave & 3, dh = KP == 1 ? wave >> 2 : 0, dl = lane;
+  // Past the slice's last group every load repeats it (and meets A rows of zeros).
+  auto gclamp = [&](int g) { return g < g1 - 1 ? g : g1 - 1; };
+  // A rows of step t by DMA: wave w copies rows 32 w .. 32 w + 31 of the step's 256 (group, row)
+  // pairs, 8 rows (1 KB) an instruction; a group past the slice's end loads zeros (outside the range)
+  const int arow = (32 * wave) % BM + (lane >> 3), akp = (32 * wave) / BM;
+  const int avoff = (arow * a.k + 8 * ((lane & 7) ^ (lane >> 4))) * 2;
+  auto dma_a = [&](int t, int buf) {
+    const int g = g0 + t * KP + akp;
+    const int lost = g < g1 ? 0 : int(0x80000000u);
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        Ab[mb][s] =
-            __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ars, aoff[mb], (64 * g + 16 * s) * 2, 0));
-#pragma unroll
-    for (int j = 0; j < kNB; ++j) load_bwords<BITS>(Bb[j], bp, nb0 + j, g, G, lane);
-    __builtin_amdgcn_sched_barrier(0);  // keep the prefetch where it is issued
+    for (int i = 0; i < 4; ++i)
+      copy_to_lds(ars, &sh.s.a[buf][32 * wave + 8 * i][0], ((i & 1 ? avoff ^ 64 : avoff) + 16 * i * a.k) | lost,
+                  128 * gclamp(g));
   };
-  // compute_group adds a group's products only when `take` (a padded step of the rotation re-reads
-  // the slice's last group and discards it), so the rotation loop has no exits mid-way.
-  auto compute_group = [&](const u32x4 (&Ab)[MB][4], const BWords (&Bb)[kNB], bool take) {
-    float16_t S[MB];
+  auto load_words = [&](TileWords<NS>& w, int t) {
+    load_tile_words<BITS, NS>(w, bp, 4 * tn + db, gclamp(g0 + t * KP + dkp), G, dl, NS == 2 ? 2 * dh : 0);
+  };
+  // bf16 bits of this lane's column scale in each of the wave's two column blocks
+  auto load_scales = [&](uint32_t (&s)[2], int t) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      s[j] = __builtin_amdgcn_raw_buffer_load_b16(bp.sc, (lane & 31) * 2,
+                                                  ((4 * tn + 2 * wn + j) * G + gclamp(g0 + t * KP + kp)) * 64, 0);
+  };
+  auto high_bits = [&](const TileWords<NS>& w) {  // of the thread's own steps
+    if constexpr (BITS == 5 && NS == 2) return w.hi.x >> (8 * dh);
+    else return w.hi.x;
+  };
+
+  float16_t C[2][2], T[2][2];  // [column block][row block]
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+      C[j][mb] = float16_t{};
+      T[j][mb] = float16_t{};
+    }
+  const float my_rs = int(threadIdx.x) < BM ? row_scale(a, m0 + threadIdx.x) : 0.0f;
+
+  TileWords<NS> wq[2];  // the words of steps t + 1 and t + 2
+  uint32_t sc[2][2];    // the scales of steps t and t + 1
+  float last_sc = 0.0f;
+  auto dequant = [&](auto sc_, int buf, const TileWords<NS>& w) {
+    constexpr int S = decltype(sc_)::value;
+    // (6-bit words of four steps keep steps 2-3 in their second high word)
+    const uint32_t hi = BITS == 6 && NS == 4 && S >= 2 ? w.hi.y : high_bits(w);
+    tile_dequant_step<BITS, NS, S>(&sh.s.b[buf][dkp][db][2 * dh + S][dl][0], w, hi, magic);
+  };
+  using i0 = std::integral_constant<int, 0>;
+  using i1 = std::integral_constant<int, 1>;
+  using i2 = std::integral_constant<int, 2>;
+  using i3 = std::integral_constant<int, 3>;
+  const int ahead = wave >= 4 ? 1 : 0;
+  auto dequant_all = [&](int buf, const TileWords<NS>& w) {
+    dequant(i0{}, buf, w);
+    dequant(i1{}, buf, w);
+    if constexpr (NS == 4) {
+      dequant(i2{}, buf, w);
+      dequant(i3{}, buf, w);
+    }
+  };
+  dma_a(0, 0);
+  dma_a(1, 1);
+  load_words(wq[0], 0);
+  load_words(wq[1], 1);
+  load_scales(sc[0], 0);
+  dequant_all(0, wq[0]);
+  if (ahead) {
+    dequant_all(1, wq[1]);
+    load_words(wq[1], 2);
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // the DMA copies of steps 0 and 1 have landed
+  __syncthreads();
+
+  auto fold = [&](int j, float s) {
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) C[j][mb][e] = __builtin_fmaf(s, T[j][mb][e], C[j][mb][e]);
+  };
+  // One step in two phases with a barrier after each: operand reads and loads, then the MFMAs with the
+  // folds and the dequantisation in their shadow. Waves 4-7 run half a step behind waves 0-3, so of a
+  // SIMD's two waves one is in each phase. Waves 0-3 dequantise step t + 1 beside the MFMAs of step t,
+  // waves 4-7 step t + 2 (ahead = 1): either is then complete when waves 0-3 start to read it, and
+  // its buffer was last read, by waves 4-7, before the first of them writes to it. The copies of a
+  // step's A rows go out two steps ahead into the buffer read a step ago. cur = t & 1 is a
+  // compile-time constant, so the register rings are indexed statically.
+  int abuf = 0;  // t mod 3: the A buffer of step t
+  // (A plain barrier: __syncthreads would wait for every copy in flight. The empty assembly keeps the
+  // compiler from moving memory accesses across it.)
+  auto phase_end = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto step = [&](int t, auto curc) {
+    constexpr int cur = decltype(curc)::value;
+    const TileWords<NS>& wnext = wq[cur ^ 1];
+    const int wbuf = cur ^ 1 ^ ahead;
+    bf16x8_t ao[4][2], bo[2][4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb) {
+        const int r = 64 * wm + 32 * mb + (lane & 31);
+        ao[s][mb] = __builtin_bit_cast(bf16x8_t, sh.s.a[abuf][kp * BM + r][(2 * s + kg) ^ ((r >> 1) & 7)]);
+      }
+      bo[0][s] = *reinterpret_cast<const bf16x8_t*>(&sh.s.b[cur][kp][2 * wn][s][lane][0]);
+    }
 #pragma unroll
     for (int s = 0; s < 4; ++s)
+      bo[1][s] = *reinterpret_cast<const bf16x8_t*>(&sh.s.b[cur][kp][2 * wn + 1][s][lane][0]);
+    __builtin_amdgcn_sched_barrier(0);
+    dma_a(t + 2, abuf == 0 ? 2 : abuf - 1);
+    // the wait at the phase's end counts the loads issued after the copies: keep that order
+    __builtin_amdgcn_sched_barrier(0);
+    load_words(wq[cur], t + 2 + ahead);
+    load_scales(sc[cur ^ 1], t + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    // the copies of step t + 1 have landed: at most the loads issued after them are in flight (vmcnt
+    // counts in order: per step the words' low nibbles, the high bits of 5- and 6-bit codes, two
+    // scales, and the four copies of step t + 2)
+    __builtin_amdgcn_s_waitcnt(BITS == 4 ? 0x0F7A : 0x0F7C);
+    phase_end();
+    __builtin_amdgcn_s_setprio(1);
+    fold(1, last_sc);  // the previous step's second column block
+    dequant(i0{}, wbuf, wnext);
+    if constexpr (NS == 4) dequant(i1{}, wbuf, wnext);
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-        S[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, Ab[mb][s]), ones,
-                                                        s == 0 ? float16_t{} : S[mb], 0, 0, 0);
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int j = 0; j < kNB; ++j) {
-      float16_t T[MB];
-      group_products<BITS, MB>(T, Ab, Bb[j], magic);
-      // a discarded group adds scale 0 times finite sums (non-finite sums already reached C from the
-      // group's own step)
-      const float sc = take ? bf16_value(uint16_t(Bb[j].scale)) : 0.0f;
+      for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          C[mb][j][e] = __builtin_fmaf(sc, __builtin_fmaf(-c0, S[mb][e], T[mb][e]), C[mb][j][e]);
+        for (int mb = 0; mb < 2; ++mb)
+          T[j][mb] =
+              __builtin_amdgcn_mfma_f32_32x32x16_bf16(ao[s][mb], bo[j][s], s == 0 ? float16_t{} : T[j][mb], 0, 0, 0);
+    fold(0, bf16_value(uint16_t(sc[cur][0])));
+    if constexpr (NS == 4) {
+      dequant(i2{}, wbuf, wnext);
+      dequant(i3{}, wbuf, wnext);
+    } else {
+      dequant(i1{}, wbuf, wnext);
     }
+    last_sc = bf16_value(uint16_t(sc[cur][1]));
+    abuf = abuf == 2 ? 0 : abuf + 1;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA,
+      __builtin_amdgcn_sched_group_barrier(0x002, NS == 4 ? 10 : 7, 0);  // then vector instructions
+    }
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // this wave's dequantised codes are in LDS
+    phase_end();
   };
-  // Loads are unconditional (past the slice end they re-read its last group, which is cached): a
-  // load under a branch makes the wait-count bookkeeping assume the worst at the join and wait for
-  // the prefetched groups too. (Every slice holds a group: the host plans splits <= k / 64.)
-  const int glast = g1 - 1;
-  auto gc = [&](int g) { return g < glast ? g : glast; };
-  // the tile's row scales (the epilogue reads them after a barrier): before any weight load is in
-  // flight, as a branch over outstanding loads would make the loop's waits conservative
-  if (threadIdx.x < kBM) sh.rs[threadIdx.x] = row_scale(a, m0 + threadIdx.x);
+  if (wave >= 4) phase_end();
+  for (int t = 0; t < steps; t += 2) {
+    step(t, i0{});
+    if (t + 1 < steps) step(t + 1, i1{});
+  }
+  if (wave < 4) phase_end();
+  fold(1, last_sc);
+  // the copies past the last step have landed and every wave is past its last operand read: LDS is
+  // free for the epilogue
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (int(threadIdx.x) < BM) sh.e.rs[threadIdx.x] = my_rs;
+
+  // ---- the K parts' sums: part 0 + part 1, through LDS
+  if constexpr (KP == 2) {
+    if (kp == 1) {
 #pragma unroll
-  for (int d = 0; d + 1 < kDepth; ++d) load_group(A[d], B[d], gc(g0 + d));
-  for (int g = g0; g < g1; g += kDepth) {
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int d = 0; d < kDepth; ++d) {
-      load_group(A[(d + kDepth - 1) % kDepth], B[(d + kDepth - 1) % kDepth], gc(g + d + kDepth - 1));
-      compute_group(A[d], B[d], g + d < g1);
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) sh.e.red[wi][(2 * j + mb) * 16 + e][lane] = C[j][mb][e];
+    }
+    __syncthreads();
+    if (kp == 1) return;  // (barriers count only the waves still running)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) C[j][mb][e] += sh.e.red[wi][(2 * j + mb) * 16 + e][lane];
+  }
+  __syncthreads();
+
+  // ---- split-K: the tile's slices in slice order, summed by the last workgroup to arrive (the
+  // hand-off of tile_finish: write-through stores, their completion, an arrival count, coherent loads)
+  if (a.splits > 1) {
+    constexpr int kSc1 = 16;                       // cache policy bit sc1
+    constexpr int kWaveBytes = 64 * 64 * 4;        // a wave's sums: [quad][lane][4 floats]
+    constexpr int kSliceBytes = 2 * WM * kWaveBytes;
+    const int tile = tn * tiles_m + tm;
+    float* part = uniform_ptr(a.ws_partials + size_t(tile) * a.splits * (kSliceBytes / 4));
+    const __amdgpu_buffer_rsrc_t prs =
+        __builtin_amdgcn_make_buffer_rsrc(part, short(0), a.splits * kSliceBytes, 0x00020000);
+    const int off = wi * kWaveBytes + lane * 16;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const u32x4 v{as_u32(C[j][mb][4 * q]), as_u32(C[j][mb][4 * q + 1]), as_u32(C[j][mb][4 * q + 2]),
+                        as_u32(C[j][mb][4 * q + 3])};
+          __builtin_amdgcn_raw_buffer_store_b128(v, prs, off + ((2 * j + mb) * 4 + q) * 1024, z * kSliceBytes, kSc1);
+        }
+    __builtin_amdgcn_s_waitcnt(0);  // the write-through stores have completed
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int old = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sh.e.last = old == a.splits - 1;
+      if (sh.e.last) __hip_atomic_store(a.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!sh.e.last) return;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb) C[j][mb] = float16_t{};
+    for (int zz = 0; zz < a.splits; ++zz) {
+      u32x4 v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(prs, off + i * 1024, zz * kSliceBytes, kSc1));
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float16_t& c = C[i >> 3][(i >> 2) & 1];
+        c[4 * (i & 3)] += as_f32(v[i].x);
+        c[4 * (i & 3) + 1] += as_f32(v[i].y);
+        c[4 * (i & 3) + 2] += as_f32(v[i].z);
+        c[4 * (i & 3) + 3] += as_f32(v[i].w);
+      }
     }
   }
-  tile_finish<MB, FUSED>(a, ap, batch, kv, sh, C, tile, z, tn, wave, lane);
+
+  // ---- epilogue: 32 rows of the wave's 64 columns at a time through LDS, then row-contiguous stores.
+  // C element e of (j, mb): row 32 mb + 8 (e / 4) + 4 kg + e % 4, column 32 j + lane % 32 of the wave.
+  float(&ot)[32][64 + 4] = sh.e.out[wave];
+  const int col0 = tn * kTileCols + 64 * wn;
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb) {
+    const int r0 = 64 * wm + 32 * mb;  // first row within the tile
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) ot[8 * (e >> 2) + 4 * kg + (e & 3)][32 * j + (lane & 31)] = C[j][mb][e];
+    if (a.kind == Q38A_EPI_RESIDUAL) {
+      // four columns per lane, four rows per instruction
+      const int c = 4 * (lane & 15), col = col0 + c;
+      float ssum[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = 4 * i + (lane >> 4), row = m0 + r0 + r;
+        const float4 y = *reinterpret_cast<const float4*>(&ot[r][c]);
+        ssum[i] = 0.0f;
+        if (row < a.m) {
+          float* res = a.residual + size_t(row) * a.n + col;
+          float x[4] = {y.x, y.y, y.z, y.w};
+          if (a.wide_out) {
+            const float4 p = *reinterpret_cast<const float4*>(res);
+            x[0] += p.x;
+            x[1] += p.y;
+            x[2] += p.z;
+            x[3] += p.w;
+            *reinterpret_cast<float4*>(res) = float4{x[0], x[1], x[2], x[3]};
+          } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              x[u] += res[u];
+              res[u] = x[u];
+            }
+          }
+          uint16_t* xb = a.xbf + size_t(row) * a.n + col;
+          if (a.wide_out)
+            *reinterpret_cast<uint2*>(xb) = uint2{uint32_t(bf16_bits(x[0])) | (uint32_t(bf16_bits(x[1])) << 16),
+                                                  uint32_t(bf16_bits(x[2])) | (uint32_t(bf16_bits(x[3])) << 16)};
+          else
+#pragma unroll
+            for (int u = 0; u < 4; ++u) xb[u] = bf16_bits(x[u]);
+          ssum[i] = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) ssum[i] += __shfl_xor(ssum[i], o, 64);
+        if ((lane & 15) == 0) sh.e.ss[wn][r0 + 4 * i + (lane >> 4)] = ssum[i];
+      }
+    } else if (a.kind == Q38A_EPI_STORE_F32) {
+      const int c = 4 * (lane & 15), col = col0 + c;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = 4 * i + (lane >> 4), row = m0 + r0 + r;
+        if (row >= a.m) continue;
+        const float rs = sh.e.rs[r0 + r];
+        const float4 y = *reinterpret_cast<const float4*>(&ot[r][c]);
+        const float x[4] = {y.x * rs, y.y * rs, y.z * rs, y.w * rs};
+        float* out = static_cast<float*>(a.out) + size_t(row) * a.ldo + col;
+        if (a.wide_out && col + 4 <= a.n_store) *reinterpret_cast<float4*>(out) = float4{x[0], x[1], x[2], x[3]};
+        else
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (col + u < a.n_store) out[u] = x[u];
+      }
+    } else {
+      // eight columns per lane, eight rows per instruction
+      const int c = 8 * (lane & 7), col = col0 + c;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 8 * i + (lane >> 3), row = m0 + r0 + r;
+        if (row >= a.m) continue;
+        const float rs = sh.e.rs[r0 + r];
+        const float4 y0 = *reinterpret_cast<const float4*>(&ot[r][c]), y1 = *reinterpret_cast<const float4*>(&ot[r][c + 4]);
+        const uint16_t x[8] = {bf16_bits(y0.x * rs), bf16_bits(y0.y * rs), bf16_bits(y0.z * rs), bf16_bits(y0.w * rs),
+                               bf16_bits(y1.x * rs), bf16_bits(y1.y * rs), bf16_bits(y1.z * rs), bf16_bits(y1.w * rs)};
+        uint16_t* out = static_cast<uint16_t*>(a.out) + size_t(row) * a.ldo + col;
+        if (a.wide_out && col + 8 <= a.n_store)
+          *reinterpret_cast<u32x4*>(out) = u32x4{uint32_t(x[0]) | (uint32_t(x[1]) << 16), uint32_t(x[2]) | (uint32_t(x[3]) << 16),
+                                                 uint32_t(x[4]) | (uint32_t(x[5]) << 16), uint32_t(x[6]) | (uint32_t(x[7]) << 16)};
+        else
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+            if (col + u < a.n_store) out[u] = x[u];
+      }
+    }
+  }
+  if (a.kind == Q38A_EPI_RESIDUAL) {
+    // the tile's 128 columns are one block of the sums of squares: its two waves' halves, in order
+    __syncthreads();
+    const int r = threadIdx.x;  // part 0's waves only: 2 WM x 64 threads >= BM
+    if (r < BM && m0 + r < a.m) a.partials_out[size_t(m0 + r) * a.norm_blocks + tn] = sh.e.ss[0][r] + sh.e.ss[1][r];
+  }
 }
 
 // ---- large M: 256 x 256 tiles, weights dequantised once per workgroup --------------------------
@@ -548,9 +862,6 @@ struct alignas(16) BigShared {
   u32x4 a[2][kBigRows][8];
   float rs[kBigRows];  // row scales of the folded RMSNorm
 };
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float float2_t __attribute__((ext_vector_type(2)));
 
 // Two dequantised codes -> packed bf16(code x scale) (RNE): x0, x1 are fp32 128 + u (u the stored
 // code), sneg = -(128 + 2^(b-1)) * scale, exact in fp32, so fma gives (u - 2^(b-1)) * scale
@@ -804,19 +1115,17 @@ struct alignas(16) GemvShared {
 
 // MERGE: the staged A is the gated merge of decode split partials (MergeIn) instead of a.a.
 template <int BITS, int EV, bool FUSED, bool MERGE>
-__global__ void __launch_bounds__(threads_of(1)) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(kGemvThreads) __attribute__((amdgpu_waves_per_eu(4)))
 qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) {
-  constexpr int kKP = kparts_of(1);
   __shared__ GemmShared sh;
   __shared__ GemvShared sv;
   const int hw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63, wave = hw % waves_of(1), kp = hw / waves_of(1);
+  const int lane = threadIdx.x & 63, wave = hw % kColWaves, kp = hw / kColWaves;
   const int kg = lane >> 5;
-  const int z = blockIdx.x % a.splits, tile = blockIdx.x / a.splits;
-  const int tn = tile % a.tiles_n, m0 = (tile / a.tiles_n) * 32;
+  const int z = blockIdx.x % a.splits, tn = blockIdx.x / a.splits, m0 = 0;
   const int G = a.k / 64;
   const int gs0 = int((long long)z * G / a.splits), gs1 = int((long long)(z + 1) * G / a.splits);
-  const int gm = gs0 + (gs1 - gs0) / kKP;  // K part 0: [gs0, gm), part 1: [gm, gs1)
+  const int gm = gs0 + (gs1 - gs0) / kKParts;  // K part 0: [gs0, gm), part 1: [gm, gs1)
   const int g0 = kp == 0 ? gs0 : gm, g1 = kp == 0 ? gm : gs1;
   const int nb = tn * (kTileN / 32) + wave;  // this wave's 32-column block
   const int valid_rows = a.m - m0 < 32 ? a.m - m0 : 32;
@@ -841,14 +1150,14 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
     u32x4 v[kStageChunks];
 #pragma unroll
     for (int i = 0; i < kStageChunks; ++i) {
-      const int c = int(threadIdx.x) + i * threads_of(1), r = c / cpr, kc = c % cpr;
+      const int c = int(threadIdx.x) + i * kGemvThreads, r = c / cpr, kc = c % cpr;
       if (c < chunks) v[i] = *reinterpret_cast<const u32x4*>(a.a + size_t(m0 + r) * a.k + 64 * gs0 + 8 * kc);
     }
     if constexpr (MERGE) {
       // four dims of one (row, q head) per step; a row that is not a decode row (n != 1) is zero
       const DecodePlan pl = wave_decode_plan(batch, mi.nkv, mi.max_splits, mi.target_items);
       const int qpr = 16 * (gs1 - gs0);  // quads per row
-      for (int c = threadIdx.x; c < valid_rows * qpr; c += threads_of(1)) {
+      for (int c = threadIdx.x; c < valid_rows * qpr; c += kGemvThreads) {
         const int r = c / qpr, kq = c % qpr, k = 64 * gs0 + 4 * kq;
         const int h = k / kHeadDim, d = k % kHeadDim, row = m0 + r;
         const int b = batch.tok_seq[row];
@@ -866,17 +1175,17 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
     const int np = valid_rows * a.norm_blocks;
 #pragma unroll
     for (int i = 0; i < kStagePartials; ++i) {
-      const int c = int(threadIdx.x) + i * threads_of(1);
+      const int c = int(threadIdx.x) + i * kGemvThreads;
       if (a.partials_in && c < np) pv[i] = a.partials_in[size_t(m0) * a.norm_blocks + c];
     }
 #pragma unroll
     for (int i = 0; i < kStageChunks; ++i) {
-      const int c = int(threadIdx.x) + i * threads_of(1), r = c / cpr, kc = c % cpr;
+      const int c = int(threadIdx.x) + i * kGemvThreads, r = c / cpr, kc = c % cpr;
       if (c < chunks) *reinterpret_cast<u32x4*>(&sv.a[r][8 * kc]) = v[i];
     }
 #pragma unroll
     for (int i = 0; i < kStagePartials; ++i) {
-      const int c = int(threadIdx.x) + i * threads_of(1);
+      const int c = int(threadIdx.x) + i * kGemvThreads;
       if (a.partials_in && c < np) sv.p[c] = pv[i];
     }
     __syncthreads();
@@ -891,7 +1200,7 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
       sh.rs[threadIdx.x] = rs;
     }
     const int ng = gs1 - gs0;
-    for (int t = threadIdx.x; t < 32 * ng; t += threads_of(1)) {
+    for (int t = threadIdx.x; t < 32 * ng; t += kGemvThreads) {
       const int gl = t >> 5, r = t & 31;
       float acc = 0.0f;
 #pragma unroll
@@ -908,8 +1217,7 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
     __syncthreads();
   }
 
-  float16_t C[1][1];
-  C[0][0] = float16_t{};
+  float16_t C = float16_t{};
   const float c0 = 128.0f + float(1 << (BITS - 1));
   const uint32_t magic = 0x43004300u;
   const int arow = lane & 31;
@@ -919,11 +1227,10 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
       load_bwords<BITS>(B[(d + kGemvDepth - 1) % kGemvDepth], bp, nb, gc(g + d + kGemvDepth - 1), G, lane);
       __builtin_amdgcn_sched_barrier(0);
       const int gl = gc(g + d) - gs0;
-      u32x4 Ab[1][4];
+      u32x4 Ab[4];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) Ab[0][s] = *reinterpret_cast<const u32x4*>(&sv.a[arow][64 * gl + 16 * s + 8 * kg]);
-      float16_t T[1];
-      group_products<BITS, 1>(T, Ab, B[d], magic);
+      for (int s = 0; s < 4; ++s) Ab[s] = *reinterpret_cast<const u32x4*>(&sv.a[arow][64 * gl + 16 * s + 8 * kg]);
+      const float16_t T = group_products<BITS>(Ab, B[d], magic);
       const float sc = g + d < g1 ? bf16_value(uint16_t(B[d].scale)) : 0.0f;
 #pragma unroll
       for (int i = 0; i < EV; ++i) {
@@ -931,7 +1238,7 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
         const float sr[4] = {sq.x, sq.y, sq.z, sq.w};
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          C[0][0][4 * i + r] = __builtin_fmaf(sc, __builtin_fmaf(-c0, sr[r], T[0][4 * i + r]), C[0][0][4 * i + r]);
+          C[4 * i + r] = __builtin_fmaf(sc, __builtin_fmaf(-c0, sr[r], T[4 * i + r]), C[4 * i + r]);
       }
     }
   }
@@ -939,14 +1246,14 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
   // part 1 hands its sums to part 0 and ends (barriers count only the waves still running)
   if (kp == 1) {
 #pragma unroll
-    for (int e = 0; e < 4 * EV; ++e) sh.kpart[wave][e][lane] = C[0][0][e];
+    for (int e = 0; e < 4 * EV; ++e) sh.kpart[wave][e][lane] = C[e];
   }
   __syncthreads();
   if (kp == 1) return;
 #pragma unroll
-  for (int e = 0; e < 4 * EV; ++e) C[0][0][e] += sh.kpart[wave][e][lane];
+  for (int e = 0; e < 4 * EV; ++e) C[e] += sh.kpart[wave][e][lane];
   __syncthreads();  // the union's other uses may overwrite kpart from here on
-  tile_finish<1, FUSED, EV>(a, ap, batch, kv, sh, C, tile, z, tn, wave, lane);
+  tile_finish<FUSED, EV>(a, ap, batch, kv, sh, C, tn, z, wave, lane);
 }
 
 // ---- decode-size M (<= 8 rows) on a wide column grid: 64-column tiles over the whole K --------------
@@ -1053,9 +1360,9 @@ __global__ void __launch_bounds__(64 * kWideWaves) qgemv_wide_kernel(GemmArgs a)
     // through the wave's LDS buffer into the operand layout: row lane % 32 (rows >= 8 repeat rows
     // 0-7; their output rows are never read), k chunk 2 s + lane / 32
     sh.a[wave][d][lane >> 3][lane & 7] = A[d];
-    u32x4 Ab[1][4];
+    u32x4 Ab[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) Ab[0][s] = sh.a[wave][d][2 * s + kg][lane & 7];
+    for (int s = 0; s < 4; ++s) Ab[s] = sh.a[wave][d][2 * s + kg][lane & 7];
     // S (the rows' sums over the group) from two 16 x 16 x 32 MFMAs against ones: MFMA row r is
     // A row 4 (r / 8) + r % 4, so that output element e of lane l is row 4 (l / 32) + e, the row of
     // C element e (rows >= 8 of the 32 x 32 output are never read)
@@ -1067,11 +1374,10 @@ __global__ void __launch_bounds__(64 * kWideWaves) qgemv_wide_kernel(GemmArgs a)
           0, 0, 0);
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      float16_t T[1];
-      group_products<BITS, 1>(T, Ab, B[d][j], magic);
+      const float16_t T = group_products<BITS>(Ab, B[d][j], magic);
       const float sc = bf16_value(uint16_t(B[d][j].scale));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) C[j][e] = __builtin_fmaf(sc, __builtin_fmaf(-c0, S[e], T[0][e]), C[j][e]);
+      for (int e = 0; e < 4; ++e) C[j][e] = __builtin_fmaf(sc, __builtin_fmaf(-c0, S[e], T[e]), C[j][e]);
     }
     if (rg[d] + 1 == chunk_begin(rc[d] + 1)) {  // the chunk's last group: its sums to its slot
       float* slot = sh.c + rc[d] * (NB * 256);
@@ -1208,45 +1514,92 @@ WidePlan plan_wide(int m, int n, int k, int kind, int cus) {
   return p;
 }
 
-// Split-K plan. Small M (qgemv_kernel, one 1024-thread workgroup per CU): slices of at most
+// Split-K plan of the small-M kernel (m <= 32, one 1024-thread workgroup per CU): slices of at most
 // kSliceG groups (the staged A), and at most as many as fill the CUs once without a second round;
-// each of the two K parts keeps a group. Larger M (qgemm_kernel): enough workgroups to stream the weights at
-// HBM speed (about two per CU), at least four groups per slice.
-struct GemmPlan {
-  int mb, tiles_m, tiles_n, splits;
+// each of the two K parts keeps a group. tiles_n = 0: the shape does not take that kernel.
+struct GemvPlan {
+  int tiles_n, splits;
 };
 
-GemmPlan plan_gemm(int m, int n, int k, int cus) {
-  GemmPlan p;
+GemvPlan plan_gemv(int m, int n, int k, int cus) {
+  GemvPlan p{0, 1};
   const int G = k / 64;
-  p.mb = m <= 32 && G >= 2 ? 1 : 2;
-  p.tiles_m = (m + 32 * p.mb - 1) / (32 * p.mb);
+  if (m > 32 || G < 2) return p;
   p.tiles_n = n / kTileN;
-  const int tiles = p.tiles_m * p.tiles_n;
-  int s = 1;
-  if (p.mb == 1) {
-    // fill the CUs, but keep about 12 groups per slice at least: a slice's fixed costs (staging,
-    // the split-K tail) cost more than idle CUs below that (measured on the o-projection: 8 slices
-    // of 12 groups 17.6 us, 12 slices of 8 groups 19.0 us)
-    const int s_min = (G + kSliceG - 1) / kSliceG, s_fill = cus / tiles, s_work = G / 12;
-    s = s_fill < s_work ? s_fill : s_work;
-    if (s < s_min) s = s_min;
-    if (s > G / kparts_of(1)) s = G / kparts_of(1);
-    if (s < s_min) s = s_min;  // (G / 2 >= ceil(G / 20) for every G >= 2)
-  } else {
-    while (tiles * s < 2 * cus && G / (2 * s) >= 4 && s < 16) s *= 2;
-  }
+  // fill the CUs, but keep about 12 groups per slice at least: a slice's fixed costs (staging, the
+  // split-K tail) cost more than idle CUs below that (measured on the o-projection: 8 slices of 12
+  // groups 17.6 us, 12 slices of 8 groups 19.0 us)
+  const int s_min = (G + kSliceG - 1) / kSliceG, s_fill = cus / p.tiles_n, s_work = G / 12;
+  int s = s_fill < s_work ? s_fill : s_work;
+  if (s < s_min) s = s_min;
+  if (s > G / kKParts) s = G / kKParts;
+  if (s < s_min) s = s_min;  // (G / 2 >= ceil(G / 20) for every G >= 2)
   p.splits = s;
   return p;
 }
 
+// Tile height and K slices of the tile kernel (one workgroup per CU).
+struct TilePlan {
+  int wm, tiles_m, tiles_n, splits;
+  size_t tiles() const { return size_t(tiles_m) * tiles_n; }
+  size_t partial_floats() const { return splits > 1 ? tiles() * splits * tile_rows(wm) * kTileCols : 0; }
+  size_t counters() const { return splits > 1 ? tiles() : 0; }
+  bool fits(const q38a_gemm_workspace& ws) const {
+    return splits == 1 || (ws.partials && ws.counters && ws.partial_floats >= partial_floats() &&
+                           ws.num_counters > 0 && size_t(ws.num_counters) >= counters());
+  }
+};
+
+// The height and slice count of the least estimated time, in us, from a sweep over both on the in-
+// and the o-projection at 48 to 2,048 rows: rounds of one workgroup per CU, each of steps of 0.92 us
+// (256 rows) or 0.95 us (128 rows, two groups), 10 us around them (first loads, epilogue) and, split,
+// 3 + 2.8 s us for the hand-off. Within 8% of the best measured choice at every size of the sweep;
+// e.g. in-projection: 128 rows 2 slices of 128-row tiles 37 us (1: 52, 4: 48), 512 rows 256-row
+// tiles 86 us (128-row tiles 109); o-projection: 512 rows 3 slices of 256-row tiles 56 us (1: 101).
+TilePlan plan_tile(int m, int n, int k, int cus, int max_splits) {
+  const int G = k / 64;
+  TilePlan best{};
+  double best_cost = 1e30;
+  for (int wm = 2; wm <= 4; wm += 2) {
+    TilePlan p{wm, (m + tile_rows(wm) - 1) / tile_rows(wm), n / kTileCols, 1};
+    for (int s = 1; s <= max_splits && s <= G; ++s) {
+      p.splits = s;
+      const size_t rounds = (p.tiles() * s + cus - 1) / cus;
+      const int steps = ((G + s - 1) / s + tile_kparts(wm) - 1) / tile_kparts(wm);
+      const double cost = rounds * (steps * (wm == 4 ? 0.92 : 0.95) + 10.0 + (s > 1 ? 3.0 + 2.8 * s : 0.0));
+      if (cost < best_cost) {
+        best = p;
+        best_cost = cost;
+      }
+    }
+  }
+  return best;
+}
+
+// Launches of fewer than two 64 x 256 tiles a CU are refused without the planned split workspace;
+// larger ones run unsplit without it (they fill the CUs anyway).
+bool tile_needs_workspace(int m, int n, int k, int cus) {
+  return ((m + 63) / 64) * (n / kTileN) < 2 * cus && k / 64 >= 8;
+}
+
+// Whether the 256 x 256 tiles of the large-M kernel fill the CUs.
+bool big_fits(int m, int n, int cus) { return m > 32 && ((m + kBigRows - 1) / kBigRows) * (n / kTileN) >= cus; }
+
 }  // namespace
 
 int gemm_workspace_size(int m, int n, int k, int cus, size_t out[2]) {
-  const GemmPlan p = plan_gemm(m, n, k, cus);
-  const size_t tiles = size_t(p.tiles_m) * p.tiles_n;
-  out[0] = p.splits > 1 ? tiles * p.splits * size_t(32 * p.mb) * kTileN : 0;
-  out[1] = p.splits > 1 ? tiles : 0;
+  out[0] = out[1] = 0;
+  const GemvPlan p = plan_gemv(m, n, k, cus);
+  if (p.tiles_n > 0) {
+    if (p.splits > 1) {
+      out[0] = size_t(p.tiles_n) * p.splits * 32 * kTileN;
+      out[1] = size_t(p.tiles_n);
+    }
+  } else if (!big_fits(m, n, cus)) {
+    const TilePlan t = plan_tile(m, n, k, cus, kTileMaxSplits);
+    out[0] = t.partial_floats();
+    out[1] = t.counters();
+  }
   // the wide-tile kernel's split partials (residual epilogue), whichever epilogue the caller uses
   const WidePlan wp = plan_wide(m, n, k, Q38A_EPI_RESIDUAL, cus);
   if (wp.tiles > 0 && wp.splits > 1) {
@@ -1257,43 +1610,49 @@ int gemm_workspace_size(int m, int n, int k, int cus, size_t out[2]) {
 }
 
 template <int BITS>
-void launch_bits(const GemmPlan& pl, bool ev1, int mode, dim3 grid, dim3 block, hipStream_t stream, const GemmArgs& g,
-                 const AppendArgs& aa, const BatchArgs& ba, const KvArgs& ka, const MergeIn& mi) {
-  if (pl.mb == 1) {
-    if (mode == 1) {
-      if (ev1) hipLaunchKernelGGL((qgemv_kernel<BITS, 1, true, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
-      else hipLaunchKernelGGL((qgemv_kernel<BITS, 4, true, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
-    } else if (mode == 2) {
-      if (ev1) hipLaunchKernelGGL((qgemv_kernel<BITS, 1, false, true>), grid, block, 0, stream, g, aa, ba, ka, mi);
-      else hipLaunchKernelGGL((qgemv_kernel<BITS, 4, false, true>), grid, block, 0, stream, g, aa, ba, ka, mi);
-    } else {
-      if (ev1) hipLaunchKernelGGL((qgemv_kernel<BITS, 1, false, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
-      else hipLaunchKernelGGL((qgemv_kernel<BITS, 4, false, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
-    }
+void launch_gemv(bool ev1, int mode, dim3 grid, hipStream_t stream, const GemmArgs& g, const AppendArgs& aa,
+                 const BatchArgs& ba, const KvArgs& ka, const MergeIn& mi) {
+  const dim3 block(kGemvThreads);
+  if (mode == 1) {
+    if (ev1) hipLaunchKernelGGL((qgemv_kernel<BITS, 1, true, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
+    else hipLaunchKernelGGL((qgemv_kernel<BITS, 4, true, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
+  } else if (mode == 2) {
+    if (ev1) hipLaunchKernelGGL((qgemv_kernel<BITS, 1, false, true>), grid, block, 0, stream, g, aa, ba, ka, mi);
+    else hipLaunchKernelGGL((qgemv_kernel<BITS, 4, false, true>), grid, block, 0, stream, g, aa, ba, ka, mi);
   } else {
-    if (mode == 1) hipLaunchKernelGGL((qgemm_kernel<BITS, true>), grid, block, 0, stream, g, aa, ba, ka, mi);
-    else hipLaunchKernelGGL((qgemm_kernel<BITS, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
+    if (ev1) hipLaunchKernelGGL((qgemv_kernel<BITS, 1, false, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
+    else hipLaunchKernelGGL((qgemv_kernel<BITS, 4, false, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
   }
 }
 
-// ap: the fused in-projection append; mi: the o-projection's A merged from decode partials (only
-// plans on the small-M kernel: the caller checks gemm_merge_fits). b: the batch of either.
+template <int BITS>
+void launch_tile(int wm, dim3 grid, hipStream_t stream, const GemmArgs& g) {
+  const dim3 block(kTileThreads);
+  if (wm == 4) hipLaunchKernelGGL((qgemm_tile_kernel<BITS, 4>), grid, block, 0, stream, g);
+  else hipLaunchKernelGGL((qgemm_tile_kernel<BITS, 2>), grid, block, 0, stream, g);
+}
+
+// ap: the in-projection append (fused, or as the launch after the GEMM); mi: the o-projection's A
+// merged from decode partials (only shapes of the small-M kernel: the caller checks
+// gemm_merge_fits). b: the batch of either.
 int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_gemm_epilogue& ep,
                  const q38a_gemm_workspace& ws, const q38a_qk_norm_rope_params* ap, const q38a_batch_desc* b,
                  const q38a_kv_cache_desc* kv, const MergeIn* mi, hipStream_t stream) {
   if (m <= 0) return Q38A_OK;
   int cus = 0;
   if (int rc = device_cu_count(&cus)) return rc;
-  const GemmPlan pl = plan_gemm(m, w.n, w.k, cus);
-  if (pl.splits > 1) {
-    const size_t tiles = size_t(pl.tiles_m) * pl.tiles_n;
-    if (!ws.partials || !ws.counters || ws.partial_floats < tiles * pl.splits * size_t(32 * pl.mb) * kTileN ||
-        size_t(ws.num_counters) < tiles)
-      return set_error(Q38A_ERR_INVALID, "qgemm: workspace too small (q38a_qgemm_workspace_size)");
+  const GemvPlan pl = plan_gemv(m, w.n, w.k, cus);
+  const char* small_ws = "qgemm: workspace too small (q38a_qgemm_workspace_size)";
+  if (pl.tiles_n > 0) {
+    if (pl.splits > 1 && (!ws.partials || !ws.counters ||
+                          ws.partial_floats < size_t(pl.tiles_n) * pl.splits * 32 * kTileN || ws.num_counters < pl.tiles_n))
+      return set_error(Q38A_ERR_INVALID, small_ws);
+    if (ep.partials_in && ep.kind != Q38A_EPI_RESIDUAL && ep.hidden / 128 > kMaxNormBlocks)
+      return set_error(Q38A_ERR_INVALID, "qgemm: hidden %d above %d for the folded norm", ep.hidden,
+                       128 * kMaxNormBlocks);
+  } else if (mi) {
+    return set_error(Q38A_ERR_INVALID, "qgemm: the merged A needs the small-M kernel");
   }
-  if (pl.mb == 1 && ep.partials_in && ep.kind != Q38A_EPI_RESIDUAL && ep.hidden / 128 > kMaxNormBlocks)
-    return set_error(Q38A_ERR_INVALID, "qgemm: hidden %d above %d for the folded norm", ep.hidden,
-                     128 * kMaxNormBlocks);
   GemmArgs g{};
   g.a = A;
   g.m = m;
@@ -1302,7 +1661,7 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
   g.lo = w.lo;
   g.hi = w.hi;
   g.scales = w.scales;
-  g.kind = ap ? kEpiFused : ep.kind;
+  g.kind = ep.kind;
   g.out = ep.out;
   g.ldo = ep.ldo;
   g.n_store = ep.n_store > 0 ? ep.n_store : w.rows;
@@ -1313,53 +1672,54 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
   g.norm_blocks = ep.kind == Q38A_EPI_RESIDUAL ? w.n / 128 : ep.hidden / 128;
   g.inv_hidden = ep.hidden > 0 ? 1.0f / float(ep.hidden) : 0.0f;
   g.eps = ep.eps;
-  g.tiles_n = pl.tiles_n;
-  g.splits = pl.splits;
   g.ws_partials = ws.partials;
   g.counters = ws.counters;
-  AppendArgs aa{};
-  BatchArgs ba{};
-  KvArgs ka{};
-  MergeIn mg{};
-  if (ap) {
-    aa = AppendArgs{ap->proj, ap->ld_proj, ap->q_norm, ap->k_norm, ap->eps, ap->num_q_heads, ap->num_kv_heads,
-                    ap->q_out, ap->attn_layer, ap->rope_cos_sin, ap->rope_rows};
-    ka = to_args(*kv);
-  }
-  if (b) ba = to_args(*b);
-  if (mi) {
-    if (pl.mb != 1) return set_error(Q38A_ERR_INVALID, "qgemm: the merged A needs the small-M kernel");
-    mg = *mi;
-  }
-  const int mode = ap ? 1 : mi ? 2 : 0;
+  // the append as a launch of its own after the GEMM into proj: the same bits as the two calls
+  auto then_append = [&]() -> int {
+    if (int rc = check_hip(hipGetLastError(), "qgemm launch")) return rc;
+    return ap ? launch_qk_norm_rope_append(*ap, *b, *kv, stream) : Q38A_OK;
+  };
   // large M: 256 x 256 tiles with the weights dequantised once per workgroup, when those tiles fill
   // the CUs. With the append requested, that GEMM and then the append launch: at these sizes the
-  // append in the per-group-epilogue kernel's column tiles costs more than the proj round trip
-  // (2,048 rows of the in-projection: 0.686 ms fused against 0.455 ms), and the result is then the
-  // same bits as the two calls made separately.
-  const int big_tiles = ((m + kBigRows - 1) / kBigRows) * (w.n / kTileN);
-  if (pl.mb == 2 && mode != 2 && big_tiles >= cus) {
-    if (mode == 1) g.kind = ep.kind;
+  // append in a GEMM's column tiles costs more than the proj round trip.
+  if (pl.tiles_n == 0 && big_fits(m, w.n, cus)) {
     g.tiles_n = w.n / kTileN;
     g.splits = 1;
-    const dim3 bgrid{unsigned(big_tiles)}, bblock{unsigned(kBigThreads)};
+    const dim3 bgrid(unsigned(((m + kBigRows - 1) / kBigRows) * g.tiles_n)), bblock{unsigned(kBigThreads)};
     switch (w.bits) {
       case 4: hipLaunchKernelGGL((qgemm_big_kernel<4>), bgrid, bblock, 0, stream, g); break;
       case 5: hipLaunchKernelGGL((qgemm_big_kernel<5>), bgrid, bblock, 0, stream, g); break;
       case 6: hipLaunchKernelGGL((qgemm_big_kernel<6>), bgrid, bblock, 0, stream, g); break;
       default: return set_error(Q38A_ERR_UNSUPPORTED, "qgemm: %d-bit weights are not supported", w.bits);
     }
-    if (int rc = check_hip(hipGetLastError(), "qgemm launch")) return rc;
-    return mode == 1 ? launch_qk_norm_rope_append(*ap, *b, *kv, stream) : Q38A_OK;
+    return then_append();
+  }
+  if (pl.tiles_n == 0) {
+    TilePlan tp = plan_tile(m, w.n, w.k, cus, kTileMaxSplits);
+    if (!tp.fits(ws)) {
+      if (tile_needs_workspace(m, w.n, w.k, cus)) return set_error(Q38A_ERR_INVALID, small_ws);
+      tp = plan_tile(m, w.n, w.k, cus, 1);
+    }
+    g.tiles_n = tp.tiles_n;
+    g.splits = tp.splits;
+    auto aligned = [](const void* p, size_t to) { return reinterpret_cast<uintptr_t>(p) % to == 0; };
+    g.wide_out = ep.kind == Q38A_EPI_RESIDUAL ? aligned(ep.residual, 16) && aligned(ep.xbf, 8)
+                                              : aligned(ep.out, 16) && ep.ldo % (ep.kind == Q38A_EPI_STORE_F32 ? 4 : 8) == 0;
+    const dim3 tgrid(unsigned(tp.tiles() * tp.splits));
+    switch (w.bits) {
+      case 4: launch_tile<4>(tp.wm, tgrid, stream, g); break;
+      case 5: launch_tile<5>(tp.wm, tgrid, stream, g); break;
+      case 6: launch_tile<6>(tp.wm, tgrid, stream, g); break;
+      default: return set_error(Q38A_ERR_UNSUPPORTED, "qgemm: %d-bit weights are not supported", w.bits);
+    }
+    return then_append();
   }
   // decode-size M on a wide weight: the wide-tile kernel (store epilogues: 64-column tiles, no
-  // split-K; residual: 128-column tiles, K split). With the append requested, that GEMM and then the
-  // append launch (the same bits as the two calls).
-  const WidePlan wp = mode == 2 ? WidePlan{0, 0, 1} : plan_wide(m, w.n, w.k, ep.kind, cus);
+  // split-K; residual: 128-column tiles, K split), then the append launch if requested.
+  const WidePlan wp = mi ? WidePlan{0, 0, 1} : plan_wide(m, w.n, w.k, ep.kind, cus);
   if (wp.tiles > 0 && (wp.splits == 1 || (ws.partials && ws.counters &&
                                           ws.partial_floats >= size_t(wp.tiles) * wp.splits * wp.nb * 256 &&
                                           ws.num_counters >= wp.tiles))) {
-    if (mode == 1) g.kind = ep.kind;
     const dim3 wgrid(unsigned(wp.tiles), unsigned(wp.splits)), wblock(64 * kWideWaves);
 #define Q38A_WIDE(B)                                                                            \
   case B:                                                                                       \
@@ -1373,22 +1733,36 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
       default: return set_error(Q38A_ERR_UNSUPPORTED, "qgemm: %d-bit weights are not supported", w.bits);
     }
 #undef Q38A_WIDE
-    if (int rc = check_hip(hipGetLastError(), "qgemm launch")) return rc;
-    return mode == 1 ? launch_qk_norm_rope_append(*ap, *b, *kv, stream) : Q38A_OK;
+    return then_append();
   }
-  const dim3 grid(unsigned(pl.tiles_m * pl.tiles_n * pl.splits)), block(unsigned(threads_of(pl.mb)));
+  AppendArgs aa{};
+  BatchArgs ba{};
+  KvArgs ka{};
+  MergeIn mg{};
+  if (ap) {
+    g.kind = kEpiFused;
+    aa = AppendArgs{ap->proj, ap->ld_proj, ap->q_norm, ap->k_norm, ap->eps, ap->num_q_heads, ap->num_kv_heads,
+                    ap->q_out, ap->attn_layer, ap->rope_cos_sin, ap->rope_rows};
+    ka = to_args(*kv);
+  }
+  if (b) ba = to_args(*b);
+  if (mi) mg = *mi;
+  g.tiles_n = pl.tiles_n;
+  g.splits = pl.splits;
+  const int mode = ap ? 1 : mi ? 2 : 0;
+  const dim3 grid(unsigned(pl.tiles_n * pl.splits));
   const bool ev1 = m <= 8;
   switch (w.bits) {
-    case 4: launch_bits<4>(pl, ev1, mode, grid, block, stream, g, aa, ba, ka, mg); break;
-    case 5: launch_bits<5>(pl, ev1, mode, grid, block, stream, g, aa, ba, ka, mg); break;
-    case 6: launch_bits<6>(pl, ev1, mode, grid, block, stream, g, aa, ba, ka, mg); break;
+    case 4: launch_gemv<4>(ev1, mode, grid, stream, g, aa, ba, ka, mg); break;
+    case 5: launch_gemv<5>(ev1, mode, grid, stream, g, aa, ba, ka, mg); break;
+    case 6: launch_gemv<6>(ev1, mode, grid, stream, g, aa, ba, ka, mg); break;
     default: return set_error(Q38A_ERR_UNSUPPORTED, "qgemm: %d-bit weights are not supported", w.bits);
   }
   return check_hip(hipGetLastError(), "qgemm launch");
 }
 
 // Whether q38a_qgemm_merge_oproj runs the merge inside the GEMM for m rows (the small-M kernel).
-bool gemm_merge_fits(int m, int n, int k, int cus) { return plan_gemm(m, n, k, cus).mb == 1; }
+bool gemm_merge_fits(int m, int n, int k, int cus) { return plan_gemv(m, n, k, cus).tiles_n > 0; }
 
 }  // namespace q38a
 
