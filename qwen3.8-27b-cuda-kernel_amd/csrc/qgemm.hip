@@ -354,6 +354,107 @@ __device__ inline float16_t group_products(const u32x4 (&Ab)[4], const BWords& b
   return T;
 }
 
+// ---- the epilogue of the tile kernels --------------------------------------------------------------
+// A wave's output goes out in blocks of 32 rows x 64 columns, each laid out by rows in the wave's LDS
+// block first, so that every store instruction covers whole 128- or 256-byte row runs.
+typedef float OutBlock[32][64 + 4];
+
+// Two MFMA outputs (columns 0-31 and 32-63) by rows: element e of a lane is row 8 (e / 4) + 4 (lane / 32)
+// + e % 4, column lane % 32.
+__device__ inline void block_to_rows(OutBlock& ot, const float16_t& left, const float16_t& right, int lane) {
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int r = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+    ot[r][lane & 31] = left[e];
+    ot[r][32 + (lane & 31)] = right[e];
+  }
+}
+
+// The block at (row0, col0): rs_of its rows' scales (store epilogues), ss its rows' sums of squares over
+// the 64 columns (residual epilogue), both in LDS.
+__device__ inline void store_block(const GemmArgs& a, const OutBlock& ot, int row0, int col0, const float* rs_of, float* ss,
+                                   int lane) {
+  if (a.kind == Q38A_EPI_RESIDUAL) {
+    // four columns per lane, four rows per instruction
+    const int c = 4 * (lane & 15), col = col0 + c;
+    float ssum[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 4 * i + (lane >> 4), row = row0 + r;
+      const float4 y = *reinterpret_cast<const float4*>(&ot[r][c]);
+      ssum[i] = 0.0f;
+      if (row < a.m) {
+        float* res = a.residual + size_t(row) * a.n + col;
+        float x[4] = {y.x, y.y, y.z, y.w};
+        if (a.wide_out) {
+          const float4 p = *reinterpret_cast<const float4*>(res);
+          x[0] += p.x;
+          x[1] += p.y;
+          x[2] += p.z;
+          x[3] += p.w;
+          *reinterpret_cast<float4*>(res) = float4{x[0], x[1], x[2], x[3]};
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            x[u] += res[u];
+            res[u] = x[u];
+          }
+        }
+        uint16_t* xb = a.xbf + size_t(row) * a.n + col;
+        if (a.wide_out)
+          *reinterpret_cast<uint2*>(xb) = uint2{uint32_t(bf16_bits(x[0])) | (uint32_t(bf16_bits(x[1])) << 16),
+                                                uint32_t(bf16_bits(x[2])) | (uint32_t(bf16_bits(x[3])) << 16)};
+        else
+#pragma unroll
+          for (int u = 0; u < 4; ++u) xb[u] = bf16_bits(x[u]);
+        ssum[i] = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1) ssum[i] += __shfl_xor(ssum[i], o, 64);
+      if ((lane & 15) == 0) ss[4 * i + (lane >> 4)] = ssum[i];
+    }
+  } else if (a.kind == Q38A_EPI_STORE_F32) {
+    const int c = 4 * (lane & 15), col = col0 + c;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 4 * i + (lane >> 4), row = row0 + r;
+      if (row >= a.m) continue;
+      const float rs = rs_of[r];
+      const float4 y = *reinterpret_cast<const float4*>(&ot[r][c]);
+      const float x[4] = {y.x * rs, y.y * rs, y.z * rs, y.w * rs};
+      float* out = static_cast<float*>(a.out) + size_t(row) * a.ldo + col;
+      if (a.wide_out && col + 4 <= a.n_store) *reinterpret_cast<float4*>(out) = float4{x[0], x[1], x[2], x[3]};
+      else
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (col + u < a.n_store) out[u] = x[u];
+    }
+  } else {
+    // eight columns per lane, eight rows per instruction
+    const int c = 8 * (lane & 7), col = col0 + c;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 8 * i + (lane >> 3), row = row0 + r;
+      if (row >= a.m) continue;
+      const float rs = rs_of[r];
+      const float4 y0 = *reinterpret_cast<const float4*>(&ot[r][c]), y1 = *reinterpret_cast<const float4*>(&ot[r][c + 4]);
+      const uint16_t x[8] = {bf16_bits(y0.x * rs), bf16_bits(y0.y * rs), bf16_bits(y0.z * rs), bf16_bits(y0.w * rs),
+                             bf16_bits(y1.x * rs), bf16_bits(y1.y * rs), bf16_bits(y1.z * rs), bf16_bits(y1.w * rs)};
+      uint16_t* out = static_cast<uint16_t*>(a.out) + size_t(row) * a.ldo + col;
+      if (a.wide_out && col + 8 <= a.n_store)
+        *reinterpret_cast<u32x4*>(out) = u32x4{uint32_t(x[0]) | (uint32_t(x[1]) << 16), uint32_t(x[2]) | (uint32_t(x[3]) << 16),
+                                               uint32_t(x[4]) | (uint32_t(x[5]) << 16), uint32_t(x[6]) | (uint32_t(x[7]) << 16)};
+      else
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (col + u < a.n_store) out[u] = x[u];
+    }
+  }
+}
+
 // ---- 33 rows and more: 256 x 128 or 128 x 128 tiles, exact codes -------------------------------
 // Eight waves of 64 x 64. The tile's columns are dequantised once per workgroup into LDS as the
 // exact signed codes in bf16 (MFMA B operand layout: block, step, lane, 8 k) and shared by the
@@ -388,7 +489,7 @@ struct alignas(16) TileShared {
     struct {  // after the K loop
       union {
         float red[4][64][64];               // the second K part's sums: [wave][element][lane]
-        float out[kTileWaves][32][64 + 4];  // 32 rows of a wave's tile
+        OutBlock out[kTileWaves];           // 32 rows of a wave's tile
       };
       float rs[tile_rows(WM)];     // row scales of the folded RMSNorm
       float ss[2][tile_rows(WM)];  // residual epilogue: each wave column's sums of squares
@@ -660,10 +761,12 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
     phase_end();
   };
   if (wave >= 4) phase_end();
-  for (int t = 0; t < steps; t += 2) {
+  int t = 0;
+  for (; t + 1 < steps; t += 2) {
     step(t, i0{});
-    if (t + 1 < steps) step(t + 1, i1{});
+    step(t + 1, i1{});
   }
+  if (t < steps) step(t, i0{});
   if (wave < 4) phase_end();
   fold(1, last_sc);
   // the copies past the last step have landed and every wave is past its last operand read: LDS is
@@ -743,96 +846,12 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
     }
   }
 
-  // ---- epilogue: 32 rows of the wave's 64 columns at a time through LDS, then row-contiguous stores.
-  // C element e of (j, mb): row 32 mb + 8 (e / 4) + 4 kg + e % 4, column 32 j + lane % 32 of the wave.
-  float(&ot)[32][64 + 4] = sh.e.out[wave];
-  const int col0 = tn * kTileCols + 64 * wn;
+  // ---- epilogue: 32 rows of the wave's 64 columns at a time through LDS
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb) {
-    const int r0 = 64 * wm + 32 * mb;  // first row within the tile
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) ot[8 * (e >> 2) + 4 * kg + (e & 3)][32 * j + (lane & 31)] = C[j][mb][e];
-    if (a.kind == Q38A_EPI_RESIDUAL) {
-      // four columns per lane, four rows per instruction
-      const int c = 4 * (lane & 15), col = col0 + c;
-      float ssum[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int r = 4 * i + (lane >> 4), row = m0 + r0 + r;
-        const float4 y = *reinterpret_cast<const float4*>(&ot[r][c]);
-        ssum[i] = 0.0f;
-        if (row < a.m) {
-          float* res = a.residual + size_t(row) * a.n + col;
-          float x[4] = {y.x, y.y, y.z, y.w};
-          if (a.wide_out) {
-            const float4 p = *reinterpret_cast<const float4*>(res);
-            x[0] += p.x;
-            x[1] += p.y;
-            x[2] += p.z;
-            x[3] += p.w;
-            *reinterpret_cast<float4*>(res) = float4{x[0], x[1], x[2], x[3]};
-          } else {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              x[u] += res[u];
-              res[u] = x[u];
-            }
-          }
-          uint16_t* xb = a.xbf + size_t(row) * a.n + col;
-          if (a.wide_out)
-            *reinterpret_cast<uint2*>(xb) = uint2{uint32_t(bf16_bits(x[0])) | (uint32_t(bf16_bits(x[1])) << 16),
-                                                  uint32_t(bf16_bits(x[2])) | (uint32_t(bf16_bits(x[3])) << 16)};
-          else
-#pragma unroll
-            for (int u = 0; u < 4; ++u) xb[u] = bf16_bits(x[u]);
-          ssum[i] = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) ssum[i] += __shfl_xor(ssum[i], o, 64);
-        if ((lane & 15) == 0) sh.e.ss[wn][r0 + 4 * i + (lane >> 4)] = ssum[i];
-      }
-    } else if (a.kind == Q38A_EPI_STORE_F32) {
-      const int c = 4 * (lane & 15), col = col0 + c;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int r = 4 * i + (lane >> 4), row = m0 + r0 + r;
-        if (row >= a.m) continue;
-        const float rs = sh.e.rs[r0 + r];
-        const float4 y = *reinterpret_cast<const float4*>(&ot[r][c]);
-        const float x[4] = {y.x * rs, y.y * rs, y.z * rs, y.w * rs};
-        float* out = static_cast<float*>(a.out) + size_t(row) * a.ldo + col;
-        if (a.wide_out && col + 4 <= a.n_store) *reinterpret_cast<float4*>(out) = float4{x[0], x[1], x[2], x[3]};
-        else
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (col + u < a.n_store) out[u] = x[u];
-      }
-    } else {
-      // eight columns per lane, eight rows per instruction
-      const int c = 8 * (lane & 7), col = col0 + c;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = 8 * i + (lane >> 3), row = m0 + r0 + r;
-        if (row >= a.m) continue;
-        const float rs = sh.e.rs[r0 + r];
-        const float4 y0 = *reinterpret_cast<const float4*>(&ot[r][c]), y1 = *reinterpret_cast<const float4*>(&ot[r][c + 4]);
-        const uint16_t x[8] = {bf16_bits(y0.x * rs), bf16_bits(y0.y * rs), bf16_bits(y0.z * rs), bf16_bits(y0.w * rs),
-                               bf16_bits(y1.x * rs), bf16_bits(y1.y * rs), bf16_bits(y1.z * rs), bf16_bits(y1.w * rs)};
-        uint16_t* out = static_cast<uint16_t*>(a.out) + size_t(row) * a.ldo + col;
-        if (a.wide_out && col + 8 <= a.n_store)
-          *reinterpret_cast<u32x4*>(out) = u32x4{uint32_t(x[0]) | (uint32_t(x[1]) << 16), uint32_t(x[2]) | (uint32_t(x[3]) << 16),
-                                                 uint32_t(x[4]) | (uint32_t(x[5]) << 16), uint32_t(x[6]) | (uint32_t(x[7]) << 16)};
-        else
-#pragma unroll
-          for (int u = 0; u < 8; ++u)
-            if (col + u < a.n_store) out[u] = x[u];
-      }
-    }
+    const int r0 = 64 * wm + 32 * mb;
+    block_to_rows(sh.e.out[wave], C[0][mb], C[1][mb], lane);
+    store_block(a, sh.e.out[wave], m0 + r0, tn * kTileCols + 64 * wn, sh.e.rs + r0, sh.e.ss[wn] + r0, lane);
   }
   if (a.kind == Q38A_EPI_RESIDUAL) {
     // the tile's 128 columns are one block of the sums of squares: its two waves' halves, in order
@@ -842,112 +861,51 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
   }
 }
 
-// ---- large M: 256 x 256 tiles, weights dequantised once per workgroup --------------------------
-// Eight waves (4 x 2) of 64 rows x 128 columns. Per 64-k group the workgroup stages its A rows and
-// dequantises its 256 columns once into LDS, the weights as bf16(code x scale) (the reference's own
-// weight rounding, qgemm.cu), laid out as the MFMA B operand (block, step, lane, 8 k); every wave
-// reads its operands with conflict-free 16-byte reads and the MFMA accumulates across groups
-// directly: no per-group epilogue, no row-sum MFMA. Each thread loads and dequantises its share of
-// the next group while the waves run the current one; one barrier per group. The tile count fills
-// the CUs, so no split-K.
+// ---- large M: 256 x 256 tiles, weights as bf16(code x scale) ------------------------------------
+// As the tiles above, with eight waves of 64 rows x 128 columns and the weights staged in LDS as
+// bf16(code x scale) (the reference's own weight rounding, qgemm.cu), so that the MFMA accumulates
+// across groups directly. A group goes in two halves of 32 k, each a memory phase (12 operand reads,
+// and the copies of A two groups ahead or the weights' loads) and a compute phase (16 MFMAs with half a
+// lane word's dequantisation, ~3 vector instructions per MFMA), waves 4-7 one phase behind. The tile
+// count fills the CUs, so no split-K.
+//
+// Bound: MFMA. 2,048 rows of the in-projection (448 tiles on 256 CUs, so 2 rounds for 1.75): see the
+// figures at the launch.
 constexpr int kBigRows = 256;
 constexpr int kBigWaves = 8;
 constexpr int kBigThreads = 64 * kBigWaves;
 
 struct alignas(16) BigShared {
-  uint16_t b[2][8][4][64][8];  // two groups of the tile's weights: [block][step][lane][k]
-  // two groups of the tile's A rows, copied by the DMA path of buffer loads (no registers): row r's
-  // 16-byte chunk c (k 8 c .. 8 c + 7) sits in slot c ^ (r % 8), so the MFMA reads of one chunk
-  // over 8 consecutive rows hit 8 different bank groups
-  u32x4 a[2][kBigRows][8];
-  float rs[kBigRows];  // row scales of the folded RMSNorm
+  union {
+    struct {
+      u32x4 a[3][kBigRows][8];       // three groups of the tile's A rows, [row][slot] as in TileShared
+      uint16_t b[2][8][4][64][8];    // two groups of the tile's weights: [block][step][lane][k]
+    } s;
+    struct {  // after the K loop
+      OutBlock out[kBigWaves];
+      float rs[kBigRows];     // row scales of the folded RMSNorm
+      float ss[4][kBigRows];  // residual epilogue: sums of squares of each 64 columns
+    } e;
+  };
 };
 
-// Two dequantised codes -> packed bf16(code x scale) (RNE): x0, x1 are fp32 128 + u (u the stored
-// code), sneg = -(128 + 2^(b-1)) * scale, exact in fp32, so fma gives (u - 2^(b-1)) * scale
-// exactly before the one rounding to bf16.
-__device__ inline uint32_t scaled_pair(float x0, float x1, float sc, float sneg) {
-  const float2_t f{__builtin_fmaf(x0, sc, sneg), __builtin_fmaf(x1, sc, sneg)};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
-}
-
-// Codes 2P and 2P + 1 of step S of a lane word (k 16 S + 8 kg + 2P + e) as fp32 128 + u.
+// As code_pair_bf16, times the column's scale: bf16(code x scale), rounded once (the fma's result, 14
+// significant bits, is exact). sc and off: the scale times the factor and the offset of even [0] and
+// odd [1] pairs.
 template <int BITS, int S, int P>
-__device__ inline void pair_codes(const BWords& b, float& y0, float& y1) {
-  constexpr int q = 4 * S + P;
-  uint32_t x0 = ((b.lo[S] << (16 - 4 * P)) & 0x000F0000u) | 0x43000000u;  // nibble at bit 4P
-  uint32_t x1 = ((b.lo[S] >> (4 * P)) & 0x000F0000u) | 0x43000000u;       // nibble at bit 16 + 4P
-  if constexpr (BITS == 5) {
-    x0 |= shr<q - 20>(b.hi.x) & 0x00100000u;
-    x1 |= shr<q - 4>(b.hi.x) & 0x00100000u;
-  }
-  if constexpr (BITS == 6) {
-    constexpr int r = 2 * (q & 7);
-    const uint32_t h = q < 8 ? b.hi.x : b.hi.y;
-    x0 |= shr<r - 20>(h) & 0x00300000u;
-    x1 |= shr<r - 4>(h) & 0x00300000u;
-  }
-  y0 = __builtin_bit_cast(float, x0);
-  y1 = __builtin_bit_cast(float, x1);
-}
-
-// The 8 codes of step S (k 16 S + 8 kg + i, i < 8) as fp32 128 + u.
-template <int BITS, int S>
-__device__ inline void step_codes(const BWords& b, float (&x)[8]) {
-  pair_codes<BITS, S, 0>(b, x[0], x[1]);
-  pair_codes<BITS, S, 1>(b, x[2], x[3]);
-  pair_codes<BITS, S, 2>(b, x[4], x[5]);
-  pair_codes<BITS, S, 3>(b, x[6], x[7]);
-}
-
-// load_bwords for a lane-dependent block: the block's part of every offset is per lane (a vector
-// offset), the group's part wave-uniform (scalar), so the buffer resource stays uniform.
-template <int BITS>
-__device__ inline void load_bwords_lane(BWords& b, const BPlanes& p, int nb, int g, int G, int l) {
-  constexpr int hb = BITS == 4 ? 0 : BITS == 5 ? 4 : 8;
-  const int unit0 = nb * G;  // this lane's block at group 0
-  b.lo = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(p.lo, (unit0 * 64 + l) * 16, g * 1024, 0));
-  if constexpr (BITS == 5)
-    b.hi = u32x2{__builtin_amdgcn_raw_buffer_load_b32(p.hi, (unit0 * 64 + l) * hb, g * 64 * hb, 0), 0u};
-  else if constexpr (BITS == 6)
-    b.hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(p.hi, (unit0 * 64 + l) * hb, g * 64 * hb, 0));
-  else b.hi = u32x2{0u, 0u};
-  b.scale = __builtin_amdgcn_raw_buffer_load_b16(p.sc, (unit0 * 32 + (l & 31)) * 2, g * 64, 0);
-}
-
-// Step S of dequant_to_lds (the group's k 16 S .. 16 S + 15 of this lane word).
-template <int BITS, int S>
-__device__ inline void dequant_step_to_lds(BigShared& sh, int buf, const BWords& b, int blk, int l) {
-  const float sc = bf16_value(uint16_t(b.scale));
-  const float sneg = -(128.0f + float(1 << (BITS - 1))) * sc;
-  float x[8];
-  step_codes<BITS, S>(b, x);
-  const u32x4 w{scaled_pair(x[0], x[1], sc, sneg), scaled_pair(x[2], x[3], sc, sneg),
-                scaled_pair(x[4], x[5], sc, sneg), scaled_pair(x[6], x[7], sc, sneg)};
-  *reinterpret_cast<u32x4*>(&sh.b[buf][blk][S][l][0]) = w;
+__device__ inline uint32_t scaled_pair_bf16(uint32_t lo, uint32_t hi, uint32_t magic, const float (&sc)[2],
+                                           const float (&off)[2]) {
+  constexpr int q = 4 * S + P, up = P & 1 ? 4 : 0;
+  uint32_t w = and_or_valu(lo, 0x000F000Fu << up, magic);
+  if constexpr (BITS == 5) w = and_or_valu(shr<q - 4 - up>(hi), 0x00100010u << up, w);
+  if constexpr (BITS == 6) w = and_or_valu(shr<2 * (q & 7) - 4 - up>(hi), 0x00300030u << up, w);
+  const half2_t h = __builtin_bit_cast(half2_t, w);
+  const float2_t x{__builtin_fmaf(float(h.x), sc[P & 1], off[P & 1]), __builtin_fmaf(float(h.y), sc[P & 1], off[P & 1])};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2_t));
 }
 
 template <int BITS>
-__device__ inline void dequant_to_lds(BigShared& sh, int buf, const BWords& b, int blk, int l) {
-  const float sc = bf16_value(uint16_t(b.scale));
-  const float sneg = -(128.0f + float(1 << (BITS - 1))) * sc;
-  auto step = [&](auto st) {
-    constexpr int S = decltype(st)::value;
-    float x[8];
-    step_codes<BITS, S>(b, x);
-    const u32x4 w{scaled_pair(x[0], x[1], sc, sneg), scaled_pair(x[2], x[3], sc, sneg),
-                  scaled_pair(x[4], x[5], sc, sneg), scaled_pair(x[6], x[7], sc, sneg)};
-    *reinterpret_cast<u32x4*>(&sh.b[buf][blk][S][l][0]) = w;
-  };
-  step(std::integral_constant<int, 0>{});
-  step(std::integral_constant<int, 1>{});
-  step(std::integral_constant<int, 2>{});
-  step(std::integral_constant<int, 3>{});
-}
-
-template <int BITS>
-__global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_eu(2)))
-qgemm_big_kernel(GemmArgs a) {
+__global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) qgemm_big_kernel(GemmArgs a) {
   __shared__ BigShared sh;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, kg = lane >> 5;
@@ -957,25 +915,40 @@ qgemm_big_kernel(GemmArgs a) {
   const int m0 = __builtin_amdgcn_readfirstlane((blockIdx.x / a.tiles_n) * kBigRows);
   const int G = a.k / 64;
   const BPlanes bp = make_bplanes<BITS>(a);
-
-  // the staging thread's half column of weights: block dblk of the tile, lane word dl
-  const int dcol = threadIdx.x & 255, dblk = dcol >> 5, dl = (dcol & 31) + 32 * (threadIdx.x >> 8);
-  const int dnb = tn * 8 + dblk;
-  // and its four 16-byte chunks of A (rows past M load as zero through the buffer's range)
+  const uint32_t magic = 0x68006800u;  // fp16 2048 in both halves
   const int valid_rows = __builtin_amdgcn_readfirstlane(a.m - m0 < kBigRows ? a.m - m0 : kBigRows);
   const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(
       uniform_ptr(const_cast<uint16_t*>(a.a) + size_t(m0) * a.k), short(0), valid_rows * a.k * int(sizeof(uint16_t)),
       0x00020000);
-  // A rows of group g into buffer buf by the DMA path: wave w copies rows 32 w .. 32 w + 31 in four
-  // 1 KB instructions (8 rows each; lane l: row 8 i + l / 8, slot l % 8, i.e. chunk (l % 8) ^ (row % 8))
+  // Loads past the last group repeat it and are not used. A rows by DMA: wave w copies rows 32 w ..
+  // 32 w + 31, 8 rows (1 KB) an instruction; rows past M load as zero through the buffer's range.
+  auto gcl = [&](int g) { return g < G - 1 ? g : G - 1; };
+  const int avoff = ((32 * wave + (lane >> 3)) * a.k + 8 * ((lane & 7) ^ (lane >> 4))) * 2;
   auto dma_a = [&](int g, int buf) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 32 * wave + 8 * i + (lane >> 3), c = (lane & 7) ^ (r & 7);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          ars, (__attribute__((address_space(3))) void*)&sh.a[buf][32 * wave + 8 * i][0], 16, (r * a.k + 8 * c) * 2,
-          128 * g, 0, 0);
-    }
+    for (int i = 0; i < 4; ++i)
+      copy_to_lds(ars, &sh.s.a[buf][32 * wave + 8 * i][0], (i & 1 ? avoff ^ 64 : avoff) + 16 * i * a.k, 128 * gcl(g));
+  };
+  // the thread's lane word of a group: block `wave` of the tile, and its column's scale
+  TileWords<4> wq[2];
+  uint32_t sq[2];
+  auto load_words = [&](int slot, int g) {
+    load_tile_words<BITS, 4>(wq[slot], bp, 8 * tn + wave, gcl(g), G, lane, 0);
+    sq[slot] = __builtin_amdgcn_raw_buffer_load_b16(bp.sc, (lane & 31) * 2, ((8 * tn + wave) * G + gcl(g)) * 64, 0);
+  };
+  auto dequant = [&](auto st, int buf, const TileWords<4>& w, const float (&sc)[2], const float (&off)[2]) {
+    constexpr int S = decltype(st)::value;
+    const uint32_t lo = w.lo[S], lo8 = lo >> 8, hi = BITS == 6 && S >= 2 ? w.hi.y : w.hi.x;
+    const u32x4 v{scaled_pair_bf16<BITS, S, 0>(lo, hi, magic, sc, off), scaled_pair_bf16<BITS, S, 1>(lo, hi, magic, sc, off),
+                  scaled_pair_bf16<BITS, S, 2>(lo8, hi, magic, sc, off), scaled_pair_bf16<BITS, S, 3>(lo8, hi, magic, sc, off)};
+    *reinterpret_cast<u32x4*>(&sh.s.b[buf][wave][S][lane][0]) = v;
+  };
+  auto factors = [&](uint32_t bits, float (&sc)[2], float (&off)[2]) {
+    const float s = bf16_value(uint16_t(bits));
+    sc[0] = s * 0.5f;
+    sc[1] = s * (1.0f / 32);
+    off[0] = s * -(1024.0f + float(1 << (BITS - 1)));
+    off[1] = s * -(64.0f + float(1 << (BITS - 1)));
   };
 
   float16_t C[2][4];
@@ -983,113 +956,123 @@ qgemm_big_kernel(GemmArgs a) {
   for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
     for (int j = 0; j < 4; ++j) C[mb][j] = float16_t{};
+  const float my_rs = threadIdx.x < kBigRows ? row_scale(a, m0 + threadIdx.x) : 0.0f;
 
-  if (threadIdx.x < kBigRows) sh.rs[threadIdx.x] = row_scale(a, m0 + threadIdx.x);
-  const int glast = G - 1;
-  auto gcl = [&](int g) { return g < glast ? g : glast; };
-  // the weights two groups ahead in registers: bq[g & 1] holds group g until its dequantisation
-  BWords bq[2];
+  using i0 = std::integral_constant<int, 0>;
+  using i1 = std::integral_constant<int, 1>;
+  using i2 = std::integral_constant<int, 2>;
+  using i3 = std::integral_constant<int, 3>;
   dma_a(0, 0);
-  load_bwords_lane<BITS>(bq[0], bp, dnb, 0, G, dl);
-  load_bwords_lane<BITS>(bq[1], bp, dnb, gcl(1), G, dl);
-  dequant_to_lds<BITS>(sh, 0, bq[0], dblk, dl);
-  __builtin_amdgcn_s_waitcnt(0);  // the DMA copies of group 0 have landed
+  dma_a(1, 1);
+  load_words(0, 0);
+  load_words(1, 1);
+  {
+    float sc[2], off[2];
+    factors(sq[0], sc, off);
+    dequant(i0{}, 0, wq[0], sc, off);
+    dequant(i1{}, 0, wq[0], sc, off);
+    dequant(i2{}, 0, wq[0], sc, off);
+    dequant(i3{}, 0, wq[0], sc, off);
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // the DMA copies of groups 0 and 1 have landed
   __syncthreads();
-  // one group: cur = g & 1 (a compile-time constant, so the register ring is indexed statically)
-  auto group = [&](int g, auto curc) {
-    constexpr int cur = decltype(curc)::value;
-    // the next group's A rows into the other buffer (read during the previous group, before its
-    // barrier), then group g + 2's weights into the registers group g held
-    dma_a(gcl(g + 1), cur ^ 1);
-    load_bwords_lane<BITS>(bq[cur], bp, dnb, gcl(g + 2), G, dl);
-    const BWords& bnext = bq[cur ^ 1];
-    auto step = [&](auto st) {
-      constexpr int s = decltype(st)::value;
-      bf16x8_t ao[2];
+
+  // One half of a group (steps 2 H and 2 H + 1): a memory and a compute phase with a barrier after each,
+  // waves 4-7 one phase behind waves 0-3. A half's operands are complete when waves 0-3 read them (the
+  // codes' same half of the group before was dequantised at least one phase earlier by either set of
+  // waves), and the buffers are free when they are written: half H of group g + 1 goes where group
+  // g - 1's half H was, last read by waves 4-7 two phases before. cur = g & 1 is a compile-time constant,
+  // so the register ring is indexed statically.
+  int abuf = 0;  // g mod 3
+  auto phase_end = [&]() {  // (as in qgemm_tile_kernel)
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto half = [&](int g, auto curc, auto hc) {
+    constexpr int cur = decltype(curc)::value, H = decltype(hc)::value;
+    bf16x8_t ao[2][2], bo[2][4];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb) {
         const int r = 64 * wm + 32 * mb + (lane & 31);
-        ao[mb] = __builtin_bit_cast(bf16x8_t, sh.a[cur][r][(2 * s + kg) ^ (r & 7)]);
+        ao[s][mb] = __builtin_bit_cast(bf16x8_t, sh.s.a[abuf][r][(2 * (2 * H + s) + kg) ^ ((r >> 1) & 7)]);
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const bf16x8_t bo = *reinterpret_cast<const bf16x8_t*>(&sh.b[cur][4 * wn + j][s][lane][0]);
+      for (int j = 0; j < 4; ++j)
+        bo[s][j] = *reinterpret_cast<const bf16x8_t*>(&sh.s.b[cur][4 * wn + j][2 * H + s][lane][0]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (H == 0) {
+      dma_a(g + 2, abuf == 0 ? 2 : abuf - 1);
+    } else {
+      load_words(cur, g + 2);
+      // the copies of group g + 1 have landed: after them went out the words of group g + 1, the
+      // copies and the words of group g + 2 (two loads a word for 4-bit codes, else three)
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(BITS == 4 ? 0x0F78 : 0x0F7A);
+    }
+    phase_end();
+    __builtin_amdgcn_s_setprio(1);
+    float sc[2], off[2];
+    factors(sq[cur ^ 1], sc, off);
+    dequant(std::integral_constant<int, 2 * H>{}, cur ^ 1, wq[cur ^ 1], sc, off);
+    dequant(std::integral_constant<int, 2 * H + 1>{}, cur ^ 1, wq[cur ^ 1], sc, off);
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb) C[mb][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ao[mb], bo, C[mb][j], 0, 0, 0);
-      }
-      // group g + 1's step s dequantised into the other buffer while these MFMAs run (past the last
-      // group: a copy nobody reads)
-      dequant_step_to_lds<BITS, s>(sh, cur ^ 1, bnext, dblk, dl);
-    };
-    step(std::integral_constant<int, 0>{});
-    step(std::integral_constant<int, 1>{});
-    step(std::integral_constant<int, 2>{});
-    step(std::integral_constant<int, 3>{});
-    // the DMA copies of group g + 1 have landed (the weight loads issued after them may still be
-    // in flight: vmcnt counts in order, three loads per lane word, two for 4-bit weights)
-    __builtin_amdgcn_s_waitcnt(BITS == 4 ? 0x0F72 : 0x0F73);
-    __syncthreads();
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+          C[mb][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ao[s][mb], bo[s][j], C[mb][j], 0, 0, 0);
+    if constexpr (H == 1) abuf = abuf == 2 ? 0 : abuf + 1;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA,
+      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // then vector instructions
+    }
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // this wave's dequantised codes are in LDS
+    phase_end();
   };
-  for (int g = 0; g < G; g += 2) {
-    group(g, std::integral_constant<int, 0>{});
-    if (g + 1 < G) group(g + 1, std::integral_constant<int, 1>{});
+  if (wave >= 4) phase_end();
+  int g = 0;
+  for (; g + 1 < G; g += 2) {
+    half(g, i0{}, i0{});
+    half(g, i0{}, i1{});
+    half(g + 1, i1{}, i0{});
+    half(g + 1, i1{}, i1{});
   }
+  if (g < G) {
+    half(g, i0{}, i0{});
+    half(g, i0{}, i1{});
+  }
+  if (wave < 4) phase_end();
+  // the copies past the last group have landed and every wave is past its last operand read
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (threadIdx.x < kBigRows) sh.e.rs[threadIdx.x] = my_rs;
+  __syncthreads();
 
-  // ---- epilogue: C element e of (mb, j): row 64 wm + 32 mb + 8 (e / 4) + 4 kg + e % 4, column
-  // 256 tn + 128 wn + 32 j + lane % 32
-  auto row_of = [&](int mb, int e) { return m0 + 64 * wm + 32 * mb + 8 * (e >> 2) + 4 * kg + (e & 3); };
-  const int col0 = tn * kTileN + 128 * wn + (lane & 31);
-  if (a.kind == Q38A_EPI_RESIDUAL) {
-    // residual += C; xbf = bf16(residual); the wave's 128 columns are one norm block: sums of
-    // squares over its 4 column blocks, then over the 32 lanes of each half
-    float ss[2][16];
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        ss[mb][e] = 0.f;
-        const int row = row_of(mb, e);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (row < a.m) {
-            const int col = col0 + 32 * j;
-            float* res = a.residual + size_t(row) * a.n + col;
-            const float x = *res + C[mb][j][e];
-            *res = x;
-            a.xbf[size_t(row) * a.n + col] = bf16_bits(x);
-            ss[mb][e] = __builtin_fmaf(x, x, ss[mb][e]);
-          }
-        }
-      }
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        float v = ss[mb][e];
-#pragma unroll
-        for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-        const int row = row_of(mb, e);
-        if ((lane & 31) == 0 && row < a.m) a.partials_out[size_t(row) * a.norm_blocks + (col0 - (lane & 31)) / 128] = v;
-      }
-    return;
-  }
-  __syncthreads();  // sh.rs
+  // ---- epilogue: blocks of 32 rows x 64 columns
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int row = row_of(mb, e);
-      if (row >= a.m) continue;
-      const float rs = sh.rs[row - m0];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int col = col0 + 32 * j;
-        if (col >= a.n_store) continue;
-        const float y = C[mb][j][e] * rs;
-        if (a.kind == Q38A_EPI_STORE_F32) static_cast<float*>(a.out)[size_t(row) * a.ldo + col] = y;
-        else static_cast<uint16_t*>(a.out)[size_t(row) * a.ldo + col] = bf16_bits(y);
-      }
+    for (int jh = 0; jh < 2; ++jh) {
+      const int r0 = 64 * wm + 32 * mb;
+      block_to_rows(sh.e.out[wave], C[mb][2 * jh], C[mb][2 * jh + 1], lane);
+      store_block(a, sh.e.out[wave], m0 + r0, tn * kTileN + 128 * wn + 64 * jh, sh.e.rs + r0, sh.e.ss[2 * wn + jh] + r0,
+                  lane);
     }
+  if (a.kind == Q38A_EPI_RESIDUAL) {
+    __syncthreads();
+    const int r = threadIdx.x & (kBigRows - 1), h = threadIdx.x / kBigRows;
+    if (m0 + r < a.m)
+      a.partials_out[size_t(m0 + r) * a.norm_blocks + 2 * tn + h] = sh.e.ss[2 * h][r] + sh.e.ss[2 * h + 1][r];
+  }
 }
 
 // ---- small M (<= 32 rows): 32 x 256 tiles, sixteen waves ---------------------------------------
@@ -1674,6 +1657,9 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
   g.eps = ep.eps;
   g.ws_partials = ws.partials;
   g.counters = ws.counters;
+  auto aligned = [](const void* p, size_t to) { return reinterpret_cast<uintptr_t>(p) % to == 0; };
+  g.wide_out = ep.kind == Q38A_EPI_RESIDUAL ? aligned(ep.residual, 16) && aligned(ep.xbf, 8)
+                                            : aligned(ep.out, 16) && ep.ldo % (ep.kind == Q38A_EPI_STORE_F32 ? 4 : 8) == 0;
   // the append as a launch of its own after the GEMM into proj: the same bits as the two calls
   auto then_append = [&]() -> int {
     if (int rc = check_hip(hipGetLastError(), "qgemm launch")) return rc;
@@ -1702,9 +1688,6 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
     }
     g.tiles_n = tp.tiles_n;
     g.splits = tp.splits;
-    auto aligned = [](const void* p, size_t to) { return reinterpret_cast<uintptr_t>(p) % to == 0; };
-    g.wide_out = ep.kind == Q38A_EPI_RESIDUAL ? aligned(ep.residual, 16) && aligned(ep.xbf, 8)
-                                              : aligned(ep.out, 16) && ep.ldo % (ep.kind == Q38A_EPI_STORE_F32 ? 4 : 8) == 0;
     const dim3 tgrid(unsigned(tp.tiles() * tp.splits));
     switch (w.bits) {
       case 4: launch_tile<4>(tp.wm, tgrid, stream, g); break;
