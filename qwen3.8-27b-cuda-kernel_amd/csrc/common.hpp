@@ -129,9 +129,6 @@ __device__ inline uint32_t wave_allreduce(uint32_t x, Op op) {
   return op(b[0], b[1]);
 }
 
-__device__ inline int wave_min_i32(int x) {
-  return int(wave_allreduce(uint32_t(x), [](uint32_t a, uint32_t b) { return uint32_t(min(int(a), int(b))); }));
-}
 __device__ inline int wave_max_i32(int x) {
   return int(wave_allreduce(uint32_t(x), [](uint32_t a, uint32_t b) { return uint32_t(max(int(a), int(b))); }));
 }

@@ -1,0 +1,60 @@
+"""The append at 8,192 rows and more (four rows per wave): bit for bit against the oracle with means of
+squares on rounding boundaries (the left-to-right replay), and against the one-row-per-wave kernel
+(taken for a proj without 16-byte alignment) for head counts and token counts that leave the last wave
+of each kind of row partly filled, with positions past the RoPE table and past the page table."""
+import numpy as np
+import pytest
+import torch
+
+import q38a
+from gpu_util import HD, LD, NQ, Batch, Pool, append_params, dev, host, paged_layout, rope_dev, stream
+from test_append_mean import boundary_row
+from test_gpu_append import run_append
+from util import assert_bits_equal, f32_to_bf16_bits, randn_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+def test_boundary_means(orc):
+    rng = np.random.default_rng(3)
+    for M in (5, 257):  # one row per wave; four rows per wave
+        proj = randn_bf16(rng, (M, LD))
+        kcol = 2 * NQ * HD
+        for m in range(0, M, 2):
+            for h in (0, 3, 23):
+                proj[m, h * HD:(h + 1) * HD] = f32_to_bf16_bits(boundary_row(rng).astype(np.float32))
+            proj[m, kcol + HD:kcol + 2 * HD] = f32_to_bf16_bits(boundary_row(rng).astype(np.float32))
+        q, q_ref, pool, pool_ref = run_append(orc, [(0, 60, M)], q38a.KV_INT8, rng, proj=proj)[:4]
+        assert_bits_equal(q, q_ref, "q fp16")
+        assert_bits_equal(pool, pool_ref, "pool bytes")
+
+
+@pytest.mark.parametrize("nq,nkv,kv_dtype", [(24, 4, q38a.KV_INT8), (7, 1, q38a.KV_INT8_VT), (9, 3, q38a.KV_BF16),
+                                             (5, 5, q38a.KV_INT8)])
+def test_rows_kernel_matches_one_row_per_wave(nq, nkv, kv_dtype):
+    rng = np.random.default_rng(nq)
+    M = -(-8192 // (nq + 2 * nkv)) + 3
+    M += 1 - M % 2
+    ld = 2 * (nq + nkv) * HD
+    n0 = M // 2
+    seqs = [(0, 33, n0), (1, 0, 1), (2, 900, M - n0 - 1)]
+    b = Batch(seqs)
+    bt, pages = paged_layout(rng, [p + n for _, p, n in seqs])
+    bt = bt[:, :-1] if bt.shape[1] > 15 else bt  # the last pages' tokens have no page: not stored
+    fill = rng.integers(0, 256, q38a.page_bytes(kv_dtype, nkv) * pages, dtype=np.uint8)
+    proj = dev(randn_bf16(rng, (M, ld)))
+    odd = torch.zeros(M * ld + 4, dtype=torch.int16, device="cuda")
+    odd[4:] = proj.view(-1)  # 8 bytes past a 16-byte boundary
+    qn, kn = dev(rng.normal(1.0, 0.2, HD).astype(np.float32)), dev(rng.normal(1.0, 0.2, HD).astype(np.float32))
+    rope = rope_dev(900 + M - n0 - 40)  # the last positions lie past the table: NaN q, nothing stored
+    got = []
+    for p in (proj, odd[4:]):
+        pool = Pool(kv_dtype, pages, bt, nkv=nkv, fill=fill)
+        q = torch.zeros(M * nq * HD, dtype=torch.int16, device="cuda")
+        print(f"append rows: nq={nq} nkv={nkv} M={M} dtype={kv_dtype}", flush=True)
+        q38a.qk_norm_rope_append(append_params(p, qn, kn, q, rope, nq=nq, nkv=nkv, ld=ld), b.desc, pool.desc, stream())
+        torch.cuda.synchronize()
+        got.append((host(q, np.uint16), pool.download()))
+    assert_bits_equal(got[0][0], got[1][0], "q")
+    assert_bits_equal(got[0][1], got[1][1], "pool bytes")
+    assert (got[0][0].reshape(M, -1)[-30:] == 0x7E00).all()
