@@ -17,7 +17,7 @@ namespace {
 template <int DT>
 __global__ void __launch_bounds__(kThreads, 2) attn_decode_kernel(DecodeArgs a, BatchArgs batch, KvArgs kv) {
   __shared__ DecodeShared<> sh;
-  const DecodePlan pl = wave_decode_plan(batch, a.nkv, a.max_splits, a.target_items);
+  const DecodePlan pl = wave_decode_plan<true>(batch, a.nkv, a.max_splits, a.target_items);
   decode_items<DT>(a, batch, kv, pl, sh, blockIdx.x, gridDim.x);
 }
 
@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(kMergeThreads) attn_merge_kernel(MergeArgs a, 
   const int hq = blockIdx.x, b = blockIdx.y;
   const int L = decode_len(batch, b);
   const int row = batch.seq_start[b];
-  const DecodePlan pl = wave_decode_plan(batch, a.nkv, a.max_splits, a.target_items);
+  const DecodePlan pl = wave_decode_plan<true>(batch, a.nkv, a.max_splits, a.target_items);
   if (L == 0) return;
   const int splits = ceil_div_i(ceil_div_i(L, kPageTokens), pl.cp);
   const float* src = a.scratch + (size_t(b) * a.nq + hq) * a.max_splits * (kHeadDim + 2);

@@ -120,7 +120,7 @@ __device__ inline int wave_max_i(int x) { return wave_max_i32(x); }
 struct DecodePlan {
   int cp;      // pages per item (wave-uniform)
   int pages0;  // pages of decode row `lane` (rows 0..63), kept so locating items rereads nothing
-  int items;   // decode items of the launch (wave-uniform)
+  int items;   // decode items of the launch (wave-uniform; not counted by a fitted plan)
 };
 
 __device__ inline int decode_pages(const BatchArgs& batch, int s) {
@@ -128,7 +128,12 @@ __device__ inline int decode_pages(const BatchArgs& batch, int s) {
 }
 
 // Pages per item of a decode launch: every row needs at most max_splits items per kv head, and the
-// batch yields about target_items items.
+// batch yields about target_items items. FIT (a grid of one workgroup per target item, each taking
+// every target-th item): not more than target_items, so that no workgroup has a second item while the
+// others are done. Each row's last item is partly filled, so whole pages of psum * nkv / target_items
+// alone overshoot the target about every sixth batch (8 rows, 203K tokens on bf16 pages: 520 items
+// of 25 pages against 512, the launch 183 us; 504 items of 26 pages, 158 us).
+template <bool FIT>
 __device__ inline DecodePlan wave_decode_plan(const BatchArgs& batch, int nkv, int max_splits, int target_items) {
   const int lane = threadIdx.x & 63;
   DecodePlan pl;
@@ -139,14 +144,33 @@ __device__ inline DecodePlan wave_decode_plan(const BatchArgs& batch, int nkv, i
     psum += p;
     pmax = max(pmax, p);
   }
-  psum = wave_sum_i(psum);
+  psum = __builtin_amdgcn_readfirstlane(wave_sum_i(psum));  // (scalars: cp must stay wave-uniform)
   pmax = wave_max_i(pmax);
   const int by_splits = ceil_div_i(pmax, max_splits);
   const int by_target = int((static_cast<long long>(psum) * nkv + target_items - 1) / target_items);
   pl.cp = __builtin_amdgcn_readfirstlane(max(1, max(by_splits, by_target)));
-  int items = ceil_div_i(pl.pages0, pl.cp);
-  for (int s0 = 64; s0 < batch.num_seqs; s0 += 64) items += ceil_div_i(decode_pages(batch, s0 + lane), pl.cp);
-  pl.items = __builtin_amdgcn_readfirstlane(wave_sum_i(items) * nkv);
+  auto count = [&]() {
+    int items = ceil_div_i(pl.pages0, pl.cp);
+    for (int s0 = 64; s0 < batch.num_seqs; s0 += 64) items += ceil_div_i(decode_pages(batch, s0 + lane), pl.cp);
+    return __builtin_amdgcn_readfirstlane(wave_sum_i(items) * nkv);
+  };
+  if constexpr (FIT) {
+    // (Counting costs a wave reduction on the way to the first loads: not where a partly filled item
+    // per row cannot reach the target. One item per row and head too many: nothing to be gained.)
+    const long long most = static_cast<long long>(psum) + static_cast<long long>(batch.num_seqs) * pl.cp;
+    if (pl.cp > 1 && most * nkv > static_cast<long long>(target_items) * pl.cp && batch.num_seqs * nkv <= target_items) {
+      // longer items in steps of the overshoot's share
+      int items = count();
+      for (int i = 0; i < 8 && items > target_items; ++i) {
+        pl.cp += max(1, int(static_cast<long long>(pl.cp) * (items - target_items) / target_items));
+        items = count();
+      }
+      pl.cp = __builtin_amdgcn_readfirstlane(pl.cp);
+    }
+    pl.items = 0;  // (not used: the kernels stride over the items until wave_locate finds none)
+  } else {
+    pl.items = count();
+  }
   return pl;
 }
 

@@ -1138,7 +1138,7 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
     }
     if constexpr (MERGE) {
       // four dims of one (row, q head) per step; a row that is not a decode row (n != 1) is zero
-      const DecodePlan pl = wave_decode_plan(batch, mi.nkv, mi.max_splits, mi.target_items);
+      const DecodePlan pl = wave_decode_plan<true>(batch, mi.nkv, mi.max_splits, mi.target_items);
       const int qpr = 16 * (gs1 - gs0);  // quads per row
       for (int c = threadIdx.x; c < valid_rows * qpr; c += kGemvThreads) {
         const int r = c / qpr, kq = c % qpr, k = 64 * gs0 + 4 * kq;

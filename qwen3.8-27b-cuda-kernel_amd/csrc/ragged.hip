@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(kRaggedThreads, 1)
                                                          qp);
     }
   } else {
-    const DecodePlan pl = wave_decode_plan(batch, d.nkv, d.max_splits, d.target_items);
+    const DecodePlan pl = wave_decode_plan<false>(batch, d.nkv, d.max_splits, d.target_items);
     const int wg = bid < r.decode_first ? bid : bid - r.prefill_blocks;
     if (wg == 0 && threadIdx.x == 0) {
       r.header[0] = pl.cp;
