@@ -653,8 +653,10 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
       C[j][mb] = float16_t{};
       T[j][mb] = float16_t{};
     }
-  TileWords<NS> wq[2];  // the words of steps t + 1 and t + 2
-  uint32_t sc[2][2];    // the scales of steps t and t + 1
+  // Words and scales go out three steps ahead (~3 us: each is read once, from HBM, by this workgroup's
+  // XCD). Slot t % 4 holds the words dequantised in step t - 1 and the scales of step t.
+  TileWords<NS> wq[4];
+  uint32_t sc[4][2];
   float last_sc = 0.0f;
   auto dequant = [&](auto sc_, int buf, const TileWords<NS>& w) {
     constexpr int S = decltype(sc_)::value;
@@ -677,15 +679,18 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
   };
   dma_a(0, 0);
   dma_a(1, 1);
-  load_words(wq[0], 0);
-  load_words(wq[1], 1);
+  TileWords<NS> first[2];
+  load_words(first[0], 0);
+  load_words(first[1], 1);
   load_scales(sc[0], 0);
-  const float my_rs = int(threadIdx.x) < BM ? row_scale(a, m0 + threadIdx.x) : 0.0f;  // (with the first loads in flight)
-  dequant_all(0, wq[0]);
-  if (ahead) {
-    dequant_all(1, wq[1]);
-    load_words(wq[1], 2);
+#pragma unroll
+  for (int i = 1; i < 4; ++i) {
+    load_words(wq[i], i + ahead);
+    if (i < 3) load_scales(sc[i], i);
   }
+  const float my_rs = int(threadIdx.x) < BM ? row_scale(a, m0 + threadIdx.x) : 0.0f;  // (with the first loads in flight)
+  dequant_all(0, first[0]);
+  if (ahead) dequant_all(1, first[1]);
   __builtin_amdgcn_s_waitcnt(0);  // the DMA copies of steps 0 and 1 have landed
   __syncthreads();
 
@@ -700,7 +705,7 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
   // SIMD's two waves one is in each phase. Waves 0-3 dequantise step t + 1 beside the MFMAs of step t,
   // waves 4-7 step t + 2 (ahead = 1): either is then complete when waves 0-3 start to read it, and
   // its buffer was last read, by waves 4-7, before the first of them writes to it. The copies of a
-  // step's A rows go out two steps ahead into the buffer read a step ago. cur = t & 1 is a
+  // step's A rows go out two steps ahead into the buffer read a step ago. cur = t % 4 is a
   // compile-time constant, so the register rings are indexed statically.
   int abuf = 0;  // t mod 3: the A buffer of step t
   // (A plain barrier: __syncthreads would wait for every copy in flight. The empty assembly keeps the
@@ -714,8 +719,8 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
   };
   auto step = [&](int t, auto curc) {
     constexpr int cur = decltype(curc)::value;
-    const TileWords<NS>& wnext = wq[cur ^ 1];
-    const int wbuf = cur ^ 1 ^ ahead;
+    const TileWords<NS>& wnext = wq[(cur + 1) & 3];
+    const int wbuf = (cur & 1) ^ 1 ^ ahead;
     bf16x8_t ao[4][2], bo[2][4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -724,17 +729,17 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
         const int r = 64 * wm + 32 * mb + (lane & 31);
         ao[s][mb] = __builtin_bit_cast(bf16x8_t, sh.s.a[abuf][kp * BM + r][(2 * s + kg) ^ ((r >> 1) & 7)]);
       }
-      bo[0][s] = *reinterpret_cast<const bf16x8_t*>(&sh.s.b[cur][kp][2 * wn][s][lane][0]);
+      bo[0][s] = *reinterpret_cast<const bf16x8_t*>(&sh.s.b[cur & 1][kp][2 * wn][s][lane][0]);
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      bo[1][s] = *reinterpret_cast<const bf16x8_t*>(&sh.s.b[cur][kp][2 * wn + 1][s][lane][0]);
+      bo[1][s] = *reinterpret_cast<const bf16x8_t*>(&sh.s.b[cur & 1][kp][2 * wn + 1][s][lane][0]);
     __builtin_amdgcn_sched_barrier(0);
     dma_a(t + 2, abuf == 0 ? 2 : abuf - 1);
     // the wait at the phase's end counts the loads issued after the copies: keep that order
     __builtin_amdgcn_sched_barrier(0);
-    load_words(wq[cur], t + 2 + ahead);
-    load_scales(sc[cur ^ 1], t + 1);
+    load_words(wq[cur], t + 4 + ahead);
+    load_scales(sc[(cur + 3) & 3], t + 3);
     __builtin_amdgcn_sched_barrier(0);
     // the copies of step t + 1 have landed: at most the loads issued after them are in flight (vmcnt
     // counts in order: per step the words' low nibbles, the high bits of 5- and 6-bit codes, two
@@ -773,11 +778,15 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
   };
   if (wave >= 4) phase_end();
   int t = 0;
-  for (; t + 1 < steps; t += 2) {
+  for (; t + 3 < steps; t += 4) {
     step(t, i0{});
     step(t + 1, i1{});
+    step(t + 2, i2{});
+    step(t + 3, i3{});
   }
   if (t < steps) step(t, i0{});
+  if (t + 1 < steps) step(t + 1, i1{});
+  if (t + 2 < steps) step(t + 2, i2{});
   if (wave < 4) phase_end();
   fold(1, last_sc);
   // the copies past the last step have landed and every wave is past its last operand read: LDS is
@@ -951,9 +960,10 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
     for (int i = 0; i < 4; ++i)
       copy_to_lds(ars, &sh.s.a[buf][32 * wave + 8 * i][0], (i & 1 ? avoff ^ 64 : avoff) + 16 * i * a.k, 128 * gcl(g));
   };
-  // the thread's lane word of a group: block `wave` of the tile, and its column's scale
-  TileWords<4> wq[2];
-  uint32_t sq[2];
+  // the thread's lane word of a group (block `wave` of the tile) and its column's scale, four groups
+  // ahead: group g in slot g % 4 until its dequantisation beside group g - 1's MFMAs
+  TileWords<4> wq[4];
+  uint32_t sq[4];
   auto load_words = [&](int slot, int g) {
     load_tile_words<BITS, 4>(wq[slot], bp, 8 * tn + wave, gcl(g), G, lane, 0);
     sq[slot] = __builtin_amdgcn_raw_buffer_load_b16(bp.sc, (lane & 31) * 2, ((8 * tn + wave) * G + gcl(g)) * 64, 0);
@@ -987,6 +997,8 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
   dma_a(1, 1);
   load_words(0, 0);
   load_words(1, 1);
+  load_words(2, 2);
+  load_words(3, 3);
   const float my_rs = threadIdx.x < kBigRows ? row_scale(a, m0 + threadIdx.x) : 0.0f;  // (with the first loads in flight)
   {
     float sc[2], off[2];
@@ -1003,7 +1015,7 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
   // waves 4-7 one phase behind waves 0-3. A half's operands are complete when waves 0-3 read them (the
   // codes' same half of the group before was dequantised at least one phase earlier by either set of
   // waves), and the buffers are free when they are written: half H of group g + 1 goes where group
-  // g - 1's half H was, last read by waves 4-7 two phases before. cur = g & 1 is a compile-time constant,
+  // g - 1's half H was, last read by waves 4-7 two phases before. cur = g % 4 is a compile-time constant,
   // so the register ring is indexed statically.
   int abuf = 0;  // g mod 3
   auto phase_end = [&]() {  // (as in qgemm_tile_kernel)
@@ -1025,24 +1037,24 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        bo[s][j] = *reinterpret_cast<const bf16x8_t*>(&sh.s.b[cur][4 * wn + j][2 * H + s][lane][0]);
+        bo[s][j] = *reinterpret_cast<const bf16x8_t*>(&sh.s.b[cur & 1][4 * wn + j][2 * H + s][lane][0]);
     }
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (H == 0) {
       dma_a(g + 2, abuf == 0 ? 2 : abuf - 1);
     } else {
-      load_words(cur, g + 2);
-      // the copies of group g + 1 have landed: after them went out the words of group g + 1, the
-      // copies and the words of group g + 2 (two loads a word for 4-bit codes, else three)
+      load_words(cur, g + 4);
+      // the copies of group g + 1 have landed: after them went out one group's words, the copies of
+      // group g + 2 and another group's words (two loads a word for 4-bit codes, else three)
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(BITS == 4 ? 0x0F78 : 0x0F7A);
     }
     phase_end();
     __builtin_amdgcn_s_setprio(1);
     float sc[2], off[2];
-    factors(sq[cur ^ 1], sc, off);
-    dequant(std::integral_constant<int, 2 * H>{}, cur ^ 1, wq[cur ^ 1], sc, off);
-    dequant(std::integral_constant<int, 2 * H + 1>{}, cur ^ 1, wq[cur ^ 1], sc, off);
+    factors(sq[(cur + 1) & 3], sc, off);
+    dequant(std::integral_constant<int, 2 * H>{}, (cur & 1) ^ 1, wq[(cur + 1) & 3], sc, off);
+    dequant(std::integral_constant<int, 2 * H + 1>{}, (cur & 1) ^ 1, wq[(cur + 1) & 3], sc, off);
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -1061,17 +1073,20 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
     phase_end();
   };
   if (wave >= 4) phase_end();
+  auto group = [&](int g, auto curc) {
+    half(g, curc, i0{});
+    half(g, curc, i1{});
+  };
   int g = 0;
-  for (; g + 1 < G; g += 2) {
-    half(g, i0{}, i0{});
-    half(g, i0{}, i1{});
-    half(g + 1, i1{}, i0{});
-    half(g + 1, i1{}, i1{});
+  for (; g + 3 < G; g += 4) {
+    group(g, i0{});
+    group(g + 1, i1{});
+    group(g + 2, i2{});
+    group(g + 3, i3{});
   }
-  if (g < G) {
-    half(g, i0{}, i0{});
-    half(g, i0{}, i1{});
-  }
+  if (g < G) group(g, i0{});
+  if (g + 1 < G) group(g + 1, i1{});
+  if (g + 2 < G) group(g + 2, i2{});
   if (wave < 4) phase_end();
   // the copies past the last group have landed and every wave is past its last operand read
   __builtin_amdgcn_s_waitcnt(0);
