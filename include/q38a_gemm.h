@@ -1,8 +1,7 @@
 /*
  * q38a GEMMs on either side of the attention path: the in-projection that produces `proj`, with
- * the q/k RMSNorm + RoPE + KV append optionally fused into its epilogue, and the o-projection
- * that consumes the attention output, with the decode split merge optionally fused into its A
- * loader. Weights are the reference's BQ format (docs/FORMAT.md section 2: b-bit codes in 64-wide
+ * the q/k RMSNorm + RoPE + KV append optionally in the same call, and the o-projection that consumes
+ * the attention output, with the decode split merge optionally fused into its A loader. Weights are the reference's BQ format (docs/FORMAT.md section 2: b-bit codes in 64-wide
  * groups along K with one bf16 scale per (row, group)), repacked once at load time into this
  * library's MFMA layout (q38a_bq_repack). Same conventions as q38a.h: device pointers, asynchronous
  * on `stream`, no allocation, int status + q38a_last_error().
@@ -82,15 +81,12 @@ int q38a_qgemm(const uint16_t* a, int m, const q38a_bq_weight* w, const q38a_gem
                const q38a_gemm_workspace* ws, void* stream);
 
 /* The attention layers' in-projection (reference model_runner.cpp:316-338: qgemm with the
- * StoreBF16 epilogue into proj, then qk_norm_rope_append) in one launch: W is the [q | gate | k | v]
- * weight (nq + nq + 2 nkv heads of 256 rows), ep a STORE_BF16 epilogue whose out is proj. The
- * epilogue stores the gate columns into proj (what attention reads) and runs the fused
- * norm / RoPE / append on the q, k and v tiles straight from LDS: q goes to append->q_out, k and v to
- * the cache; the q, k and v columns of proj are not written. With more than 32 rows, or up to 8 on a
- * weight wide enough for the 64-column tiles, the call instead runs the GEMM into proj (every column)
- * and then the append launch, which is faster there. Either way the results are bit-identical to
- * q38a_qgemm followed by q38a_qk_norm_rope_append (append->proj and ld_proj must describe ep->out).
- * No counterpart in the reference (the producer side of the attention path). */
+ * StoreBF16 epilogue into proj, then qk_norm_rope_append) in one call: W is the [q | gate | k | v]
+ * weight (nq + nq + 2 nkv heads of 256 rows), ep a STORE_BF16 epilogue whose out is proj. Runs the GEMM
+ * into proj and then the append launch on it: the same bits as q38a_qgemm followed by
+ * q38a_qk_norm_rope_append (append->proj and ld_proj must describe ep->out). Callers may rely on the
+ * gate columns of proj, which attention reads, q_out and the cache; the q, k and v columns of proj are
+ * unspecified. No counterpart in the reference (the producer side of the attention path). */
 int q38a_qgemm_qkv_append(const uint16_t* a, int m, const q38a_bq_weight* w, const q38a_gemm_epilogue* ep,
                           const q38a_gemm_workspace* ws, const q38a_qk_norm_rope_params* append,
                           const q38a_batch_desc* batch, const q38a_kv_cache_desc* kv, void* stream);
@@ -103,14 +99,13 @@ int q38a_qgemm_qkv_append(const uint16_t* a, int m, const q38a_bq_weight* w, con
 int q38a_qgemm_merge_oproj(const q38a_attention_params* attn, const q38a_batch_desc* batch, const q38a_bq_weight* w,
                            const q38a_gemm_epilogue* ep, const q38a_gemm_workspace* ws, void* stream);
 
-/* As q38a_qgemm_merge_oproj, but for batches the small-M GEMM kernel takes (up to 32 rows) the merge
- * runs inside the GEMM's A staging and attn->out is not written (reference OPTIMIZATION_PLAN.md:202-203,
- * "attention split-merge into the o-projection's A loader"); larger batches as q38a_qgemm_merge_oproj.
- * The merged A rows are the merge kernel's bits, but the GEMM is the split-K kernel, so at <= 8 rows
- * (where q38a_qgemm takes the wide-tile kernel) the results differ from q38a_qgemm_merge_oproj's in
- * the fp32 summation order (both within the GEMM's tolerance of the exact product). Measured slower
- * than the two launches at batch 8 (every GEMM workgroup repeats the merge of its A rows), so it is
- * not the default. */
+/* As q38a_qgemm_merge_oproj, but for batches of up to 32 rows the merge runs inside the A staging of a
+ * split-K GEMM and attn->out is not written (reference OPTIMIZATION_PLAN.md:202-203, "attention
+ * split-merge into the o-projection's A loader"); larger batches as q38a_qgemm_merge_oproj. The merged A
+ * rows are the merge kernel's bits, but the GEMM is another kernel than q38a_qgemm takes, so the results
+ * differ from q38a_qgemm_merge_oproj's in the fp32 summation order (both within the GEMM's tolerance of
+ * the exact product). Measured slower than the two launches at batch 8 (every GEMM workgroup repeats the
+ * merge of its A rows), so it is not the default. */
 int q38a_qgemm_merge_oproj_in_loader(const q38a_attention_params* attn, const q38a_batch_desc* batch,
                                      const q38a_bq_weight* w, const q38a_gemm_epilogue* ep,
                                      const q38a_gemm_workspace* ws, void* stream);

@@ -1,6 +1,5 @@
-// Device code of the fused q/k offset-RMSNorm + partial RoPE + KV append, shared by the append
-// launch (append.hip) and the in-projection GEMM's fused epilogue (qgemm.hip). See append.hip for
-// the semantics and the exactness argument.
+// Device code of the fused q/k offset-RMSNorm + partial RoPE + KV append (append.hip, which has the
+// semantics and the exactness argument): the steps shared by its kernels and the one-row-per-wave form.
 #pragma once
 
 #include "common.hpp"

@@ -1,34 +1,33 @@
-// BQ-weight GEMM for gfx950 (q38a_qgemm) and the attention in-projection with the q/k norm, RoPE
-// and KV append fused into its epilogue (q38a_qgemm_qkv_append).
+// BQ-weight GEMM for gfx950 (q38a_qgemm), the attention in-projection with its q/k norm, RoPE and KV
+// append (q38a_qgemm_qkv_append: the GEMM into proj, then the append launch) and the o-projection
+// behind split decode (q38a_qgemm_merge_oproj).
 //
 // Semantics follow reference src/kernels/qgemm.cu:285-384 (epilogues) and :573-616 (launcher):
 // C[M][N] = A[M][K] . W^T, W[n][k] = code * scale[n][k / 64], A bf16, fp32 accumulation; StoreBF16
 // stores bf16(C * rs) with the folded-RMSNorm row scale rs, Residual adds C into the fp32 residual
 // stream and refreshes its bf16 copy and its per-128-column sums of squares.
 //
-// MI355X design:
-//   * v_mfma_f32_32x32x16_bf16 with the activations as the A operand and the weights as B. A lane
-//     of the B operand holds eight consecutive k of one column; the repacked weights
-//     (bq_repack.cpp) give it those codes as one 16-byte word per 64-k group (+ the high bits).
-//   * Up to 32 rows the codes enter the MFMA as the exact bf16 values 128 + u (u = the stored unsigned
-//     code, two bit operations per pair), so no conversion arithmetic is spent on them; the offset and
-//     the per-(column, group) scale are applied once per group in fp32:
+// MI355X design: v_mfma_f32_32x32x16_bf16 with the activations as the A operand and the weights as B.
+// A lane of the B operand holds eight consecutive k of one column; the repacked weights (bq_repack.cpp)
+// give it those codes as one 16-byte word per 64-k group (+ the high bits). A kernel per range of M:
+//   * up to 8 rows on a wide weight or with the residual epilogue (qgemv_wide_kernel) and up to 64
+//     (qgemm_small_kernel) a launch is a stream of weights: each wave dequantises its own columns'
+//     words in registers. The codes enter the MFMA as the exact bf16 values 128 + u (u = the stored
+//     unsigned code, two bit operations per pair); the offset and the per-(column, group) scale are
+//     applied once per group in fp32:
 //       C += scale[n][g] * (T_g - (128 + 2^(b-1)) * S_g),  T_g = sum_{k in g} a[m][k] (128 + u),
-//     where S_g = sum_{k in g} a[m][k] comes from one more MFMA against a ones operand (its output
-//     lands in the same registers as T's rows). T carries at most ~8 bits of cancellation; the
-//     result keeps ~16 significant bits, far below the bf16 output's rounding. With more rows a
-//     workgroup dequantises its columns once into LDS, for up to 1,024 rows or so as the exact signed
-//     codes (the scale still in fp32, once per group), beyond as bf16(code x scale).
-//   * Small M leaves too few tiles to pull the weights at HBM speed, so K is split over several
-//     workgroups: each writes its fp32 partial tile (rows < M only) with write-through stores,
-//     counts its arrival on a per-tile counter, and the last to arrive sums the slices in slice
-//     order (deterministic) and runs the epilogue, then resets the counter.
-//   * The fused in-projection tiles are exactly one 256-column head: a q, k or v tile is rounded to
-//     bf16 into LDS and the append's per-row code (append.hpp) runs on it, so q/k/v never make the
-//     round trip through proj; gate tiles are stored to proj, where attention reads them.
+//     S_g = sum_{k in g} a[m][k] from MFMAs of A against a constant. T carries at most ~8 bits of
+//     cancellation; the result keeps ~16 significant bits, far below the bf16 output's rounding.
+//   * beyond, a workgroup dequantises its columns once into LDS for all its rows: up to about 1,000
+//     rows (qgemm_tile_kernel) as the exact signed codes, the scale still in fp32 once per group; where
+//     256 x 256 tiles fill the CUs (qgemm_big_kernel) as bf16(code x scale), the reference's rounding.
+//   * where tiles leave CUs idle, K is split over several workgroups: each writes its fp32 partial tile
+//     with write-through stores, counts its arrival on a per-tile counter, and the last to arrive sums
+//     the slices in slice order (deterministic) and runs the epilogue, then resets the counter.
+//   * the o-projection's A merged in the loader has a split-K kernel of its own (qgemv_kernel).
 #include <type_traits>
 
-#include "append.hpp"
+#include "common.hpp"
 #include "decode.hpp"
 #include "q38a_gemm.h"
 
@@ -41,14 +40,13 @@ int launch_qk_norm_rope_append(const q38a_qk_norm_rope_params& p, const q38a_bat
 
 namespace {
 
-// A workgroup of the small-M kernel covers 32 rows x 256 columns: two sets (K parts) of 8 waves of
+// A workgroup of the merging split-K kernel covers 32 rows x 256 columns: two sets (K parts) of 8 waves of
 // one 32-column block, each set over half the slice's groups (twice the weight bytes in flight per
 // CU), their sums added through LDS.
 constexpr int kTileN = 256;
 constexpr int kColWaves = kTileN / 32;
 constexpr int kKParts = 2;
 constexpr int kGemvThreads = 64 * kColWaves * kKParts;
-constexpr int kEpiFused = 100;  // epilogue kind of the fused in-projection
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -197,22 +195,19 @@ __device__ inline float row_scale(const GemmArgs& a, int row) {
 
 struct alignas(16) GemmShared {
   union {
-    uint16_t tile[32][kTileN + 8];   // fused epilogue: the bf16 head tile (rows x 256)
     float resid_ss[kColWaves][32];   // residual epilogue: per-wave sums of squares of its columns
     float kpart[kColWaves][16][64];  // the second K part's sums
   };
-  double stage[kColWaves][kHeadDim];  // the append's sequential-sum fallback
   float rs[32];                       // row scales of the folded RMSNorm (1 without partials_in)
   int last;
 };
 
-// The small-M kernel's end: split-K slices summed by the last workgroup to arrive, then the epilogue.
+// The merging split-K kernel's end: split-K slices summed by the last workgroup to arrive, then the epilogue.
 // C element e in this lane: row 8 (e / 4) + 4 (lane / 32) + e % 4, column 32 wave + lane % 32 of the
 // tile. Every wave of the column tile calls it (K-part waves have ended); sh.rs holds the rows' scales.
 // EQ: row quads of the MFMA output that can hold rows < M (the split-K traffic skips the others).
-template <bool FUSED, int EQ>
-__device__ void tile_finish(const GemmArgs& a, const AppendArgs& ap, const BatchArgs& batch, const KvArgs& kv,
-                            GemmShared& sh, float16_t& C, int tn, int z, int wave, int lane) {
+template <int EQ>
+__device__ void tile_finish(const GemmArgs& a, GemmShared& sh, float16_t& C, int tn, int z, int wave, int lane) {
   constexpr int kRows = 32;
   const int kg = lane >> 5;
   auto row_of = [&](int e) { return 8 * (e >> 2) + 4 * kg + (e & 3); };
@@ -279,34 +274,7 @@ __device__ void tile_finish(const GemmArgs& a, const AppendArgs& ap, const Batch
   float rs[16];
 #pragma unroll
   for (int e = 0; e < 16; ++e) rs[e] = sh.rs[row_of(e)];
-  if constexpr (FUSED) {
-    const int head = tn;  // proj column blocks: q heads, gate heads, k heads, v heads
-    const int nq = ap.nq, nkv = ap.nkv;
-    const bool is_gate = head >= nq && head < 2 * nq;
-    if (is_gate) {
-      uint16_t* out = static_cast<uint16_t*>(a.out);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = row_of(e);
-        if (row < a.m) out[size_t(row) * a.ldo + col] = bf16_bits(C[e] * rs[e]);
-      }
-      return;
-    }
-    // q / k / v head: the bf16 tile (exactly what proj would hold) into LDS, then the append rows
-#pragma unroll
-    for (int e = 0; e < 16; ++e) sh.tile[row_of(e)][32 * wave + (lane & 31)] = bf16_bits(C[e] * rs[e]);
-    __syncthreads();
-    const int rtype = head < nq ? head : (head < 2 * nq + nkv ? nq + (head - 2 * nq) : nq + nkv + (head - 2 * nq - nkv));
-    for (int r = wave; r < kRows && r < a.m; r += kColWaves) {
-      RowLoads L;
-      L.m = r;
-      L.r = rtype;
-      L.pos = batch.tok_pos[L.m];
-      L.raw = *reinterpret_cast<const uint2*>(&sh.tile[r][4 * lane]);
-      row_meta(ap, batch, kv, lane, L);
-      append_row(ap, kv, sh.stage[wave], lane, L);
-    }
-  } else if (a.kind == Q38A_EPI_RESIDUAL) {
+  if (a.kind == Q38A_EPI_RESIDUAL) {
     // residual += C; xbf = bf16(residual); sums of squares per 128 columns (reference
     // qgemm.cu:356-380; the sum's order differs): the 32 lanes of each half wave, then the four
     // waves of each 128-column block in wave order
@@ -1112,7 +1080,7 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
   }
 }
 
-// ---- small M (<= 32 rows): 32 x 256 tiles, sixteen waves ---------------------------------------
+// ---- the o-projection of up to 32 rows with the merge in its A staging: 32 x 256 tiles, sixteen waves
 // A decode step's rows are few, so the launch is a stream of weights: per CU as many weight bytes
 // in flight as registers allow. The workgroup's A slice (its rows x the slice's k) and the rows'
 // group sums S_g are staged in LDS once; waves keep only weight words in their register pipeline
@@ -1124,7 +1092,6 @@ constexpr int kSliceG = 20;                 // most 64-k groups in a workgroup's
 constexpr int kSliceStride = 64 * kSliceG + 8;  // bf16 per staged A row (+16 B against bank conflicts)
 
 constexpr int kMaxNormBlocks = 64;  // folded-norm partials per row (hidden <= 8192)
-constexpr int kStageChunks = (32 * 8 * kSliceG + 1023) / 1024;      // A chunks per thread
 constexpr int kStagePartials = (32 * kMaxNormBlocks + 1023) / 1024;  // partials per thread
 
 struct alignas(16) GemvShared {
@@ -1133,22 +1100,22 @@ struct alignas(16) GemvShared {
   float p[32 * kMaxNormBlocks];  // the rows' folded-norm partials
 };
 
-// MERGE: the staged A is the gated merge of decode split partials (MergeIn) instead of a.a.
-template <int BITS, int EV, bool FUSED, bool MERGE>
+// The staged A is the gated merge of decode split partials (MergeIn).
+template <int BITS, int EV>
 __global__ void __launch_bounds__(kGemvThreads) __attribute__((amdgpu_waves_per_eu(4)))
-qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) {
+qgemv_kernel(GemmArgs a, BatchArgs batch, MergeIn mi) {
   __shared__ GemmShared sh;
   __shared__ GemvShared sv;
   const int hw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, wave = hw % kColWaves, kp = hw / kColWaves;
   const int kg = lane >> 5;
-  const int z = blockIdx.x % a.splits, tn = blockIdx.x / a.splits, m0 = 0;
+  const int z = blockIdx.x % a.splits, tn = blockIdx.x / a.splits;
   const int G = a.k / 64;
   const int gs0 = int((long long)z * G / a.splits), gs1 = int((long long)(z + 1) * G / a.splits);
   const int gm = gs0 + (gs1 - gs0) / kKParts;  // K part 0: [gs0, gm), part 1: [gm, gs1)
   const int g0 = kp == 0 ? gs0 : gm, g1 = kp == 0 ? gm : gs1;
   const int nb = tn * (kTileN / 32) + wave;  // this wave's 32-column block
-  const int valid_rows = a.m - m0 < 32 ? a.m - m0 : 32;
+  const int valid_rows = a.m;  // <= 32
   const BPlanes bp = make_bplanes<BITS>(a);
 
   // B pipeline first, then the staging loads, so one round trip covers them all; loads past the
@@ -1165,21 +1132,12 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
   // MFMA output row depends on its A row only, and rows >= M are never stored) and the partials
   // of the folded norm
   {
-    const int cpr = 8 * (gs1 - gs0);  // chunks per row
-    const int chunks = MERGE ? 0 : valid_rows * cpr;
-    u32x4 v[kStageChunks];
-#pragma unroll
-    for (int i = 0; i < kStageChunks; ++i) {
-      const int c = int(threadIdx.x) + i * kGemvThreads, r = c / cpr, kc = c % cpr;
-      if (c < chunks) v[i] = *reinterpret_cast<const u32x4*>(a.a + size_t(m0 + r) * a.k + 64 * gs0 + 8 * kc);
-    }
-    if constexpr (MERGE) {
-      // four dims of one (row, q head) per step; a row that is not a decode row (n != 1) is zero
+    {  // four dims of one (row, q head) per step; a row that is not a decode row (n != 1) is zero
       const DecodePlan pl = wave_decode_plan<true>(batch, mi.nkv, mi.max_splits, mi.target_items);
       const int qpr = 16 * (gs1 - gs0);  // quads per row
       for (int c = threadIdx.x; c < valid_rows * qpr; c += kGemvThreads) {
         const int r = c / qpr, kq = c % qpr, k = 64 * gs0 + 4 * kq;
-        const int h = k / kHeadDim, d = k % kHeadDim, row = m0 + r;
+        const int h = k / kHeadDim, d = k % kHeadDim, row = r;
         const int b = batch.tok_seq[row];
         const int L = decode_len(batch, b);
         uint16_t y[4] = {0, 0, 0, 0};
@@ -1196,12 +1154,7 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
 #pragma unroll
     for (int i = 0; i < kStagePartials; ++i) {
       const int c = int(threadIdx.x) + i * kGemvThreads;
-      if (a.partials_in && c < np) pv[i] = a.partials_in[size_t(m0) * a.norm_blocks + c];
-    }
-#pragma unroll
-    for (int i = 0; i < kStageChunks; ++i) {
-      const int c = int(threadIdx.x) + i * kGemvThreads, r = c / cpr, kc = c % cpr;
-      if (c < chunks) *reinterpret_cast<u32x4*>(&sv.a[r][8 * kc]) = v[i];
+      if (a.partials_in && c < np) pv[i] = a.partials_in[c];
     }
 #pragma unroll
     for (int i = 0; i < kStagePartials; ++i) {
@@ -1273,7 +1226,7 @@ qgemv_kernel(GemmArgs a, AppendArgs ap, BatchArgs batch, KvArgs kv, MergeIn mi) 
 #pragma unroll
   for (int e = 0; e < 4 * EV; ++e) C[e] += sh.kpart[wave][e][lane];
   __syncthreads();  // the union's other uses may overwrite kpart from here on
-  tile_finish<FUSED, EV>(a, ap, batch, kv, sh, C, tn, z, wave, lane);
+  tile_finish<EV>(a, sh, C, tn, z, wave, lane);
 }
 
 // ---- decode-size M (<= 8 rows) on a wide column grid: 64-column tiles over the whole K --------------
@@ -1507,6 +1460,231 @@ __global__ void __launch_bounds__(64 * kWideWaves) qgemv_wide_kernel(GemmArgs a)
   }
 }
 
+// ---- 9 to 64 rows: the columns' weights straight into the MFMA operands ---------------------------
+// Eight waves of (32 RB rows) x 64 columns over shares of K: CW column waves x 8 / CW K parts. A wave
+// streams its weights from HBM into registers (every weight is dequantised once, by the wave whose
+// columns it is, so they are not staged) and copies its A rows, which all workgroups share, from the
+// L2 into an LDS buffer of its own, both one group ahead. (A rows loaded straight into the operand
+// layout touched four times the cache lines: 24 instead of 20.7 us at 32 rows, 34 at 64.) Codes as bf16 128 + u; the group's products start from -(128 + 2^(b-1)) times the rows'
+// sums (four more MFMAs of A against a constant, shared by the two column blocks), so T is A . codes
+// and a group costs one fma per output. The K parts' sums meet in LDS in part order; with a K split over
+// workgroups (CW = 2) the last to arrive adds the slices in slice order.
+//
+// Bound: the weight stream and, around it, one round trip of first loads and the sums' way through
+// LDS. In-projection: 9 rows 24.3 -> 16.8 us with the append, 64 rows 36 -> 26.8; o-projection:
+// 16 rows 21.9 -> 14.1, 64 rows 33 -> 22.3.
+constexpr int kSmallWaves = 8;
+constexpr int kSmallThreads = 64 * kSmallWaves;
+constexpr int kSmallMaxRows = 64;
+constexpr int kSmallMaxSplits = 8;
+
+template <int RB>
+struct alignas(16) SmallShared {
+  union {
+    u32x4 a[kSmallWaves][2][32 * RB][8];       // per wave: two groups' A rows, [row][slot] as in TileShared
+    float part[kSmallWaves][RB * 2 * 16][64];  // the waves' sums: [row block, column block, element][lane]
+    OutBlock out[2 * RB];                      // [column wave][row block]
+  };
+  float rs[32 * RB];     // row scales of the folded RMSNorm
+  float ss[2][32 * RB];  // residual epilogue: each column wave's sums of squares
+  int last;
+};
+
+template <int BITS, int RB, int CW>
+__global__ void __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(2))) qgemm_small_kernel(GemmArgs a) {
+  constexpr int KW = kSmallWaves / CW, kCols = 64 * CW;
+  constexpr int kVals = CW * RB * 2 * 16 * 64 / kSmallThreads;  // outputs per thread
+  __shared__ SmallShared<RB> sh;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, kg = lane >> 5;
+  const int cw = wave % CW, kw = wave / CW;
+  const int tn = blockIdx.x, z = blockIdx.y, Z = gridDim.y;
+  const int G = a.k / 64;
+  const int gb = z * G / Z, ge = (z + 1) * G / Z;
+  const int g0 = gb + kw * (ge - gb) / KW, g1 = gb + (kw + 1) * (ge - gb) / KW;
+  const int nb0 = tn * (kCols / 32) + 2 * cw;
+  const BPlanes bp = make_bplanes<BITS>(a);
+  const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(
+      uniform_ptr(const_cast<uint16_t*>(a.a)), short(0), a.m * a.k * int(sizeof(uint16_t)), 0x00020000);
+  // A rows of a group by DMA into the wave's own LDS buffer, 8 rows (1 KB) an instruction; rows past M
+  // fall outside the buffer's range and load as zero
+  const int avoff = ((lane >> 3) * a.k + 8 * ((lane & 7) ^ (lane >> 4))) * 2;
+  const uint32_t magic = 0x43004300u;  // bf16 128 in both halves
+  bf16x8_t neg;                        // -(128 + 2^(b-1)), exact in bf16
+#pragma unroll
+  for (int i = 0; i < 8; ++i) neg[i] = __bf16(-(128.0f + float(1 << (BITS - 1))));
+
+  float16_t C[RB][2];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) C[rb][0] = C[rb][1] = float16_t{};
+  BWords B[2][2];
+  // unconditional loads (past the share's end they repeat its last group, cached and unused): a load
+  // under a branch would make the loop's waits conservative
+  auto load_group = [&](int d, int g) {
+    const int gc = g < g1 - 1 ? g : (g1 > g0 ? g1 - 1 : gb);
+    __builtin_amdgcn_sched_barrier(0);  // (the buffer's operand reads have returned: their MFMAs are issued)
+#pragma unroll
+    for (int i = 0; i < 4 * RB; ++i)
+      copy_to_lds(ars, &sh.a[wave][d][8 * i][0], (i & 1 ? avoff ^ 64 : avoff) + 16 * i * a.k, 128 * gc);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) load_bwords<BITS, kNonTemporal>(B[d][j], bp, nb0 + j, gc, G, lane);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto compute = [&](int d) {
+    // this group's copies have landed: at most the next group's loads are in flight
+    constexpr int kNext = 4 * RB + 2 * (BITS == 4 ? 2 : 3);
+    static_assert(kNext < 16, "vmcnt's low field");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | kNext);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 A[RB][4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const int r = 32 * rb + (lane & 31);
+        A[rb][s] = sh.a[wave][d][r][(2 * s + kg) ^ ((r >> 1) & 7)];
+      }
+    float16_t N[RB];  // the products' start
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+        N[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, A[rb][s]), neg,
+                                                        s == 0 ? float16_t{} : N[rb], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float16_t T[RB];
+      auto t_step = [&](auto st) {
+        constexpr int s = decltype(st)::value;
+        const bf16x8_t bo = b_operand<BITS, s>(B[d][j], magic);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          T[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, A[rb][s]), bo,
+                                                          s == 0 ? N[rb] : T[rb], 0, 0, 0);
+      };
+      t_step(std::integral_constant<int, 0>{});
+      t_step(std::integral_constant<int, 1>{});
+      t_step(std::integral_constant<int, 2>{});
+      t_step(std::integral_constant<int, 3>{});
+      const float sc = bf16_value(uint16_t(B[d][j].scale));
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) C[rb][j][e] = __builtin_fmaf(sc, T[rb][e], C[rb][j][e]);
+    }
+  };
+  load_group(0, g0);
+  if (int(threadIdx.x) < 32 * RB) sh.rs[threadIdx.x] = row_scale(a, threadIdx.x);  // (with the first loads in flight)
+  int g = g0;
+  for (; g + 1 < g1; g += 2) {
+    load_group(1, g + 1);
+    compute(0);
+    load_group(0, g + 2);
+    compute(1);
+  }
+  if (g < g1) {
+    load_group(1, g + 1);  // (the wait in compute counts a following group's loads)
+    compute(0);
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // no copy in flight: LDS takes the sums
+  __syncthreads();
+
+  // ---- the K parts' sums in part order: value x = t + 512 i is (column wave, row block, column block,
+  // element, lane)
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sh.part[kw * CW + cw][(2 * rb + j) * 16 + e][lane] = C[rb][j][e];
+  __syncthreads();
+  float v[kVals];
+#pragma unroll
+  for (int i = 0; i < kVals; ++i) {
+    const int x = int(threadIdx.x) + kSmallThreads * i, w = x / (RB * 2 * 16 * 64), r = x % (RB * 2 * 16 * 64);
+    float y = 0.0f;
+#pragma unroll
+    for (int q = 0; q < KW; ++q) y += (&sh.part[q * CW + w][0][0])[r];
+    v[i] = y;
+  }
+  if (Z > 1) {
+    // the tile's slices (the hand-off of tile_finish)
+    constexpr int kSc1 = 16, kSlice = kVals * kSmallThreads;  // floats
+    float* part = uniform_ptr(a.ws_partials + size_t(tn) * Z * kSlice);
+#pragma unroll
+    for (int i = 0; i < kVals; ++i)
+      __hip_atomic_store(part + z * kSlice + threadIdx.x + kSmallThreads * i, v[i], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0);  // the write-through stores have completed
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int old = __hip_atomic_fetch_add(a.counters + tn, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sh.last = old == Z - 1;
+      if (sh.last) __hip_atomic_store(a.counters + tn, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!sh.last) return;
+    const __amdgpu_buffer_rsrc_t prs =
+        __builtin_amdgcn_make_buffer_rsrc(part, short(0), Z * kSlice * int(sizeof(float)), 0x00020000);
+    float V[kSmallMaxSplits][kVals];
+#pragma unroll
+    for (int q = 0; q < kSmallMaxSplits; ++q)
+#pragma unroll
+      for (int i = 0; i < kVals; ++i) {
+        const int zz = q < Z ? q : Z - 1;  // past the last slice: re-read it, not added
+        V[q][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                prs, (int(threadIdx.x) + kSmallThreads * i) * 4, zz * kSlice * 4, kSc1));
+      }
+#pragma unroll
+    for (int i = 0; i < kVals; ++i) {
+      float y = 0.0f;
+#pragma unroll
+      for (int q = 0; q < kSmallMaxSplits; ++q) y = q < Z ? y + V[q][i] : y;
+      v[i] = y;
+    }
+  }
+  __syncthreads();  // the sums' slots have been read
+#pragma unroll
+  for (int i = 0; i < kVals; ++i) {
+    const int x = int(threadIdx.x) + kSmallThreads * i, l = x & 63, e = (x >> 6) & 15, j = (x >> 10) & 1;
+    const int rb = (x >> 11) % RB, w = x / (RB * 2048);
+    sh.out[w * RB + rb][8 * (e >> 2) + 4 * (l >> 5) + (e & 3)][32 * j + (l & 31)] = v[i];
+  }
+  __syncthreads();
+  if (wave < CW * RB) {
+    const int w = wave / RB, rb = wave % RB;
+    store_block(a, sh.out[wave], 32 * rb, tn * kCols + 64 * w, sh.rs + 32 * rb, sh.ss[w] + 32 * rb, lane);
+  }
+  if (CW == 2 && a.kind == Q38A_EPI_RESIDUAL) {
+    __syncthreads();
+    const int r = threadIdx.x;
+    if (r < 32 * RB && r < a.m) a.partials_out[size_t(r) * a.norm_blocks + tn] = sh.ss[0][r] + sh.ss[1][r];
+  }
+}
+
+// Column waves, tiles and K slices of the 9- to 64-row kernel. 64-column tiles over the whole K where they
+// fill three quarters of the CUs and the epilogue allows it (the sums of squares of the residual one
+// need 128 columns), otherwise 128-column tiles with K split to fill the CUs, at least a group per wave.
+struct SmallPlan {
+  int cw, tiles, splits;
+  size_t partial_floats(int m) const {
+    return splits > 1 ? size_t(tiles) * splits * (m > 32 ? 64 : 32) * 64 * cw : 0;
+  }
+};
+
+SmallPlan plan_small(int m, int n, int k, int kind, int cus) {
+  if (kind != Q38A_EPI_RESIDUAL && n / 64 >= (3 * cus) / 4) return SmallPlan{1, n / 64, 1};
+  SmallPlan p{2, n / 128, 1};
+  const int G = k / 64;
+  int s = cus / p.tiles;
+  if (s > kSmallMaxSplits) s = kSmallMaxSplits;
+  if (s > G / 4) s = G / 4;
+  p.splits = s < 1 ? 1 : s;
+  return p;
+}
+
 // The wide-tile plan of a GEMM, or tiles = 0 when the shape does not take it: decode-size M, a
 // store epilogue on a weight wide enough to fill the CUs with 64-column tiles (no split-K), or the
 // residual epilogue on 128-column tiles with K split to fill the CUs.
@@ -1534,7 +1712,7 @@ WidePlan plan_wide(int m, int n, int k, int kind, int cus) {
   return p;
 }
 
-// Split-K plan of the small-M kernel (m <= 32, one 1024-thread workgroup per CU): slices of at most
+// Split-K plan of the merging kernel (m <= 32, one 1024-thread workgroup per CU): slices of at most
 // kSliceG groups (the staged A), and at most as many as fill the CUs once without a second round;
 // each of the two K parts keeps a group. tiles_n = 0: the shape does not take that kernel.
 struct GemvPlan {
@@ -1571,11 +1749,11 @@ struct TilePlan {
 };
 
 // The height and slice count of the least estimated time, in us, from a sweep over both on the in-
-// and the o-projection at 48 to 2,048 rows: rounds of one workgroup per CU, each of steps of 0.92 us
-// (256 rows) or 0.95 us (128 rows, two groups), 10 us around them (first loads, epilogue) and, split,
-// 3 + 2.8 s us for the hand-off. Within 8% of the best measured choice at every size of the sweep;
-// e.g. in-projection: 128 rows 2 slices of 128-row tiles 37 us (1: 52, 4: 48), 512 rows 256-row
-// tiles 86 us (128-row tiles 109); o-projection: 512 rows 3 slices of 256-row tiles 56 us (1: 101).
+// and the o-projection at 48 to 2,048 rows: rounds of one workgroup per CU, each of steps of 0.9 us
+// (256 rows) or 1.12 us (128 rows, two groups), 12 us around them (first loads, epilogue) and, split,
+// 5 + 3 s us for the hand-off. Within 6% of the best measured choice at every size of the sweep;
+// e.g. in-projection: 128 rows 2 slices of 128-row tiles 38 us (1: 53, 4: 53), 384 rows 256-row
+// tiles 83 us (128-row tiles 109); o-projection: 256 rows 3 slices of 128-row tiles 43 us (1: 72).
 TilePlan plan_tile(int m, int n, int k, int cus, int max_splits) {
   const int G = k / 64;
   TilePlan best{};
@@ -1586,7 +1764,7 @@ TilePlan plan_tile(int m, int n, int k, int cus, int max_splits) {
       p.splits = s;
       const size_t rounds = (p.tiles() * s + cus - 1) / cus;
       const int steps = ((G + s - 1) / s + tile_kparts(wm) - 1) / tile_kparts(wm);
-      const double cost = rounds * (steps * (wm == 4 ? 0.92 : 0.95) + 10.0 + (s > 1 ? 3.0 + 2.8 * s : 0.0));
+      const double cost = rounds * (steps * (wm == 4 ? 0.9 : 1.12) + 12.0 + (s > 1 ? 5.0 + 3.0 * s : 0.0));
       if (cost < best_cost) {
         best = p;
         best_cost = cost;
@@ -1615,12 +1793,21 @@ int gemm_workspace_size(int m, int n, int k, int cus, size_t out[2]) {
       out[0] = size_t(p.tiles_n) * p.splits * 32 * kTileN;
       out[1] = size_t(p.tiles_n);
     }
-  } else if (!big_fits(m, n, cus)) {
+  } else if (m > kSmallMaxRows && !big_fits(m, n, cus)) {
     const TilePlan t = plan_tile(m, n, k, cus, kTileMaxSplits);
     out[0] = t.partial_floats();
     out[1] = t.counters();
   }
-  // the wide-tile kernel's split partials (residual epilogue), whichever epilogue the caller uses
+  // whichever epilogue the caller uses: the 9- to 64-row kernel's and the wide-tile kernel's slices
+  if (m <= kSmallMaxRows) {
+    for (const int kind : {Q38A_EPI_STORE_BF16, Q38A_EPI_RESIDUAL}) {
+      const SmallPlan sp = plan_small(m, n, k, kind, cus);
+      if (sp.splits > 1) {
+        out[0] = std::max(out[0], sp.partial_floats(m));
+        out[1] = std::max(out[1], size_t(sp.tiles));
+      }
+    }
+  }
   const WidePlan wp = plan_wide(m, n, k, Q38A_EPI_RESIDUAL, cus);
   if (wp.tiles > 0 && wp.splits > 1) {
     out[0] = std::max(out[0], size_t(wp.tiles) * wp.splits * wp.nb * 256);
@@ -1630,18 +1817,21 @@ int gemm_workspace_size(int m, int n, int k, int cus, size_t out[2]) {
 }
 
 template <int BITS>
-void launch_gemv(bool ev1, int mode, dim3 grid, hipStream_t stream, const GemmArgs& g, const AppendArgs& aa,
-                 const BatchArgs& ba, const KvArgs& ka, const MergeIn& mi) {
+void launch_gemv(bool ev1, dim3 grid, hipStream_t stream, const GemmArgs& g, const BatchArgs& ba, const MergeIn& mi) {
   const dim3 block(kGemvThreads);
-  if (mode == 1) {
-    if (ev1) hipLaunchKernelGGL((qgemv_kernel<BITS, 1, true, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
-    else hipLaunchKernelGGL((qgemv_kernel<BITS, 4, true, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
-  } else if (mode == 2) {
-    if (ev1) hipLaunchKernelGGL((qgemv_kernel<BITS, 1, false, true>), grid, block, 0, stream, g, aa, ba, ka, mi);
-    else hipLaunchKernelGGL((qgemv_kernel<BITS, 4, false, true>), grid, block, 0, stream, g, aa, ba, ka, mi);
+  if (ev1) hipLaunchKernelGGL((qgemv_kernel<BITS, 1>), grid, block, 0, stream, g, ba, mi);
+  else hipLaunchKernelGGL((qgemv_kernel<BITS, 4>), grid, block, 0, stream, g, ba, mi);
+}
+
+template <int BITS>
+void launch_small(int m, int cw, dim3 grid, hipStream_t stream, const GemmArgs& g) {
+  const dim3 block(kSmallThreads);
+  if (m > 32) {
+    if (cw == 1) hipLaunchKernelGGL((qgemm_small_kernel<BITS, 2, 1>), grid, block, 0, stream, g);
+    else hipLaunchKernelGGL((qgemm_small_kernel<BITS, 2, 2>), grid, block, 0, stream, g);
   } else {
-    if (ev1) hipLaunchKernelGGL((qgemv_kernel<BITS, 1, false, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
-    else hipLaunchKernelGGL((qgemv_kernel<BITS, 4, false, false>), grid, block, 0, stream, g, aa, ba, ka, mi);
+    if (cw == 1) hipLaunchKernelGGL((qgemm_small_kernel<BITS, 1, 1>), grid, block, 0, stream, g);
+    else hipLaunchKernelGGL((qgemm_small_kernel<BITS, 1, 2>), grid, block, 0, stream, g);
   }
 }
 
@@ -1652,7 +1842,7 @@ void launch_tile(int wm, dim3 grid, hipStream_t stream, const GemmArgs& g) {
   else hipLaunchKernelGGL((qgemm_tile_kernel<BITS, 2>), grid, block, 0, stream, g);
 }
 
-// ap: the in-projection append (fused, or as the launch after the GEMM); mi: the o-projection's A
+// ap: the in-projection append (the launch after the GEMM); mi: the o-projection's A
 // merged from decode partials (only shapes of the small-M kernel: the caller checks
 // gemm_merge_fits). b: the batch of either.
 int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_gemm_epilogue& ep,
@@ -1704,9 +1894,8 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
     return ap ? launch_qk_norm_rope_append(*ap, *b, *kv, stream) : Q38A_OK;
   };
   // large M: 256 x 256 tiles with the weights dequantised once per workgroup, when those tiles fill
-  // the CUs. With the append requested, that GEMM and then the append launch: at these sizes the
-  // append in a GEMM's column tiles costs more than the proj round trip.
-  if (pl.tiles_n == 0 && big_fits(m, w.n, cus)) {
+  // the CUs
+  if (m > kSmallMaxRows && big_fits(m, w.n, cus)) {
     g.tiles_n = w.n / kTileN;
     g.splits = 1;
     const dim3 bgrid(unsigned(((m + kBigRows - 1) / kBigRows) * g.tiles_n)), bblock{unsigned(kBigThreads)};
@@ -1718,7 +1907,7 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
     }
     return then_append();
   }
-  if (pl.tiles_n == 0) {
+  if (m > kSmallMaxRows) {
     TilePlan tp = plan_tile(m, w.n, w.k, cus, kTileMaxSplits);
     if (!tp.fits(ws)) {
       if (tile_needs_workspace(m, w.n, w.k, cus)) return set_error(Q38A_ERR_INVALID, small_ws);
@@ -1736,7 +1925,7 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
     return then_append();
   }
   // decode-size M on a wide weight: the wide-tile kernel (store epilogues: 64-column tiles, no
-  // split-K; residual: 128-column tiles, K split), then the append launch if requested.
+  // split-K; residual: 128-column tiles, K split)
   const WidePlan wp = mi ? WidePlan{0, 0, 1} : plan_wide(m, w.n, w.k, ep.kind, cus);
   if (wp.tiles > 0 && (wp.splits == 1 || (ws.partials && ws.counters &&
                                           ws.partial_floats >= size_t(wp.tiles) * wp.splits * wp.nb * 256 &&
@@ -1756,27 +1945,31 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
 #undef Q38A_WIDE
     return then_append();
   }
-  AppendArgs aa{};
-  BatchArgs ba{};
-  KvArgs ka{};
-  MergeIn mg{};
-  if (ap) {
-    g.kind = kEpiFused;
-    aa = AppendArgs{ap->proj, ap->ld_proj, ap->q_norm, ap->k_norm, ap->eps, ap->num_q_heads, ap->num_kv_heads,
-                    ap->q_out, ap->attn_layer, ap->rope_cos_sin, ap->rope_rows};
-    ka = to_args(*kv);
+  if (!mi) {
+    SmallPlan sp = plan_small(m, w.n, w.k, ep.kind, cus);
+    if (sp.splits > 1 && (!ws.partials || !ws.counters || ws.partial_floats < sp.partial_floats(m) || ws.num_counters < sp.tiles)) {
+      if (pl.tiles_n == 0 && tile_needs_workspace(m, w.n, w.k, cus)) return set_error(Q38A_ERR_INVALID, small_ws);
+      sp.splits = 1;
+    }
+    const dim3 sgrid(unsigned(sp.tiles), unsigned(sp.splits));
+    switch (w.bits) {
+      case 4: launch_small<4>(m, sp.cw, sgrid, stream, g); break;
+      case 5: launch_small<5>(m, sp.cw, sgrid, stream, g); break;
+      case 6: launch_small<6>(m, sp.cw, sgrid, stream, g); break;
+      default: return set_error(Q38A_ERR_UNSUPPORTED, "qgemm: %d-bit weights are not supported", w.bits);
+    }
+    return then_append();
   }
-  if (b) ba = to_args(*b);
-  if (mi) mg = *mi;
+  // the merged A: the split-K kernel, whose staging merges
+  const BatchArgs ba = to_args(*b);
   g.tiles_n = pl.tiles_n;
   g.splits = pl.splits;
-  const int mode = ap ? 1 : mi ? 2 : 0;
   const dim3 grid(unsigned(pl.tiles_n * pl.splits));
   const bool ev1 = m <= 8;
   switch (w.bits) {
-    case 4: launch_gemv<4>(ev1, mode, grid, stream, g, aa, ba, ka, mg); break;
-    case 5: launch_gemv<5>(ev1, mode, grid, stream, g, aa, ba, ka, mg); break;
-    case 6: launch_gemv<6>(ev1, mode, grid, stream, g, aa, ba, ka, mg); break;
+    case 4: launch_gemv<4>(ev1, grid, stream, g, ba, *mi); break;
+    case 5: launch_gemv<5>(ev1, grid, stream, g, ba, *mi); break;
+    case 6: launch_gemv<6>(ev1, grid, stream, g, ba, *mi); break;
     default: return set_error(Q38A_ERR_UNSUPPORTED, "qgemm: %d-bit weights are not supported", w.bits);
   }
   return check_hip(hipGetLastError(), "qgemm launch");
