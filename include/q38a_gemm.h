@@ -111,7 +111,7 @@ int q38a_qgemm_merge_oproj_in_loader(const q38a_attention_params* attn, const q3
                                      const q38a_gemm_workspace* ws, void* stream);
 
 /* Floats of split-K partials and counters q38a_qgemm / q38a_qgemm_qkv_append may use for an
- * (m, n, k) problem: out[0] partial floats, out[1] counters. */
+ * problem of up to m rows on an (n, k) weight: out[0] partial floats, out[1] counters. */
 int q38a_qgemm_workspace_size(int m, int n, int k, size_t out[2]);
 
 #ifdef __cplusplus

@@ -132,7 +132,7 @@ __device__ inline int decode_pages(const BatchArgs& batch, int s) {
 // every target-th item): not more than target_items, so that no workgroup has a second item while the
 // others are done. Each row's last item is partly filled, so whole pages of psum * nkv / target_items
 // alone overshoot the target about every sixth batch (8 rows, 203K tokens on bf16 pages: 520 items
-// of 25 pages against 512, the launch 183 us; 504 items of 26 pages, 158 us).
+// of 25 pages against 512, the step 190 us; 504 items of 26 pages, 160 us).
 template <bool FIT>
 __device__ inline DecodePlan wave_decode_plan(const BatchArgs& batch, int nkv, int max_splits, int target_items) {
   const int lane = threadIdx.x & 63;

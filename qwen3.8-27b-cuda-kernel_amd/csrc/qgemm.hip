@@ -435,7 +435,7 @@ __device__ inline void store_block(const GemmArgs& a, const OutBlock& ot, int ro
   }
 }
 
-// ---- 33 rows and more: 256 x 128 or 128 x 128 tiles, exact codes -------------------------------
+// ---- 65 rows and more: 256 x 128 or 128 x 128 tiles, exact codes -------------------------------
 // Eight waves of 64 x 64. The tile's columns are dequantised once per workgroup into LDS as the
 // exact signed codes in bf16 (MFMA B operand layout: block, step, lane, 8 k) and shared by the
 // waves of its rows; A rows come by the DMA path of buffer loads, 16-byte chunk c of a row in
@@ -443,14 +443,15 @@ __device__ inline void store_block(const GemmArgs& a, const OutBlock& ot, int ro
 // quads of the 64 banks. Each 64-k group's products accumulate in their own registers (T, starting from
 // zero) and C += scale * T in fp32 when the group is done: the codes are exact, so the only
 // roundings are the fp32 sums'. One column block's T is folded while the other block's MFMAs run,
-// and the last one's at the start of the next step, under the latency of that step's first operand
-// reads. KP: 64-k groups per step. With 256 rows a step is one group; with 128 rows two sets of four
-// waves take one group each (the same 512 dequantised codes per step and thread, the same LDS),
-// and the sets' sums are added through LDS at the end (set 0 + set 1).
+// and the last one's beside the next step's first MFMAs. KP: 64-k groups per step. With 256 rows a step
+// is one group; with 128 rows two sets of four waves take one group each, and the sets' sums are added through LDS at the end (set 0 + set 1).
 //
-// Bound: per 64 x 64 x 64 wave step 512 MFMA cycles against 64 folds + 56 (5-bit, 256 rows) or 112
-// dequantisation instructions of 4 cycles each, i.e. the VALU, which two waves per SIMD overlap with
-// the MFMA pipe.
+// Bound: the VALU beside the MFMA. Per 64 x 64 x 64 wave step 16 MFMAs (512 cycles) against 64 folds
+// and 50 (5-bit codes, 256 rows) or 100 dequantisation instructions; two waves per SIMD hide about six
+// vector instructions per MFMA (measured, register-only loops). In-projection at 512 rows, GEMM alone:
+// 84 us, 0.9 us a step and ~10 us around them (897 TFLOP/s; hipBLASLt's plain bf16 product 90 us), against
+// 216 us of the kernel before, which read both operands from global memory in every wave; 100 us with
+// all waves in step, 93 with slot c ^ (row % 8).
 constexpr int kTileWaves = 8;
 constexpr int kTileThreads = 64 * kTileWaves;
 constexpr int kTileCols = 128;  // two waves wide
@@ -868,8 +869,8 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
 // lane word's dequantisation, ~3 vector instructions per MFMA), waves 4-7 one phase behind. The tile
 // count fills the CUs, so no split-K.
 //
-// Bound: MFMA. 2,048 rows of the in-projection (448 tiles on 256 CUs, so 2 rounds for 1.75): see the
-// figures at the launch.
+// Bound: MFMA, at the clock the card holds under it. In-projection at 2,048 rows (448 tiles on 256 CUs: 2
+// rounds for 1.75): 301 -> 265 us against the form with all waves in step and 2-byte stores (1,136 TFLOP/s; hipBLASLt's plain bf16 product 245-256 us).
 constexpr int kBigRows = 256;
 constexpr int kBigWaves = 8;
 constexpr int kBigThreads = 64 * kBigWaves;
@@ -1700,11 +1701,7 @@ WidePlan plan_wide(int m, int n, int k, int kind, int cus) {
     if (n / 64 >= (3 * cus) / 4 && wide_chunks(2, G) >= kWideWaves) p = WidePlan{2, n / 64, 1};
   } else if (n % 128 == 0) {
     const int tiles = n / 128;
-#ifdef WKS
-    int s = WKS;
-#else
     int s = cus / tiles;
-#endif
     if (s > kWideMaxSplits) s = kWideMaxSplits;
     while (s > 1 && wide_chunks(4, G / s) < kWideWaves) --s;
     if (s >= 1 && tiles * s >= cus / 2 && wide_chunks(4, G / s) >= kWideWaves) p = WidePlan{4, tiles, s};
@@ -1785,33 +1782,28 @@ bool big_fits(int m, int n, int cus) { return m > 32 && ((m + kBigRows - 1) / kB
 
 }  // namespace
 
+// Enough for every epilogue and every number of rows up to m, so that the workspace of a caller's
+// largest launch serves the smaller ones too (a launch's own plan is not monotonic in m).
 int gemm_workspace_size(int m, int n, int k, int cus, size_t out[2]) {
   out[0] = out[1] = 0;
-  const GemvPlan p = plan_gemv(m, n, k, cus);
-  if (p.tiles_n > 0) {
-    if (p.splits > 1) {
-      out[0] = size_t(p.tiles_n) * p.splits * 32 * kTileN;
-      out[1] = size_t(p.tiles_n);
-    }
-  } else if (m > kSmallMaxRows && !big_fits(m, n, cus)) {
-    const TilePlan t = plan_tile(m, n, k, cus, kTileMaxSplits);
-    out[0] = t.partial_floats();
-    out[1] = t.counters();
+  auto need = [&](size_t floats, size_t counters) {
+    out[0] = std::max(out[0], floats);
+    out[1] = std::max(out[1], counters);
+  };
+  if (m <= 0) return Q38A_OK;
+  const GemvPlan p = plan_gemv(1, n, k, cus);  // the same for every m <= 32
+  if (p.tiles_n > 0 && p.splits > 1) need(size_t(p.tiles_n) * p.splits * 32 * kTileN, size_t(p.tiles_n));
+  const WidePlan wp = plan_wide(1, n, k, Q38A_EPI_RESIDUAL, cus);  // the same for every m <= kWideRows
+  if (wp.tiles > 0 && wp.splits > 1) need(size_t(wp.tiles) * wp.splits * wp.nb * 256, size_t(wp.tiles));
+  const int ms = m < kSmallMaxRows ? m : kSmallMaxRows;  // (its partials grow with m)
+  for (const int kind : {Q38A_EPI_STORE_BF16, Q38A_EPI_RESIDUAL}) {
+    const SmallPlan sp = plan_small(ms, n, k, kind, cus);
+    if (sp.splits > 1) need(sp.partial_floats(ms), size_t(sp.tiles));
   }
-  // whichever epilogue the caller uses: the 9- to 64-row kernel's and the wide-tile kernel's slices
-  if (m <= kSmallMaxRows) {
-    for (const int kind : {Q38A_EPI_STORE_BF16, Q38A_EPI_RESIDUAL}) {
-      const SmallPlan sp = plan_small(m, n, k, kind, cus);
-      if (sp.splits > 1) {
-        out[0] = std::max(out[0], sp.partial_floats(m));
-        out[1] = std::max(out[1], size_t(sp.tiles));
-      }
-    }
-  }
-  const WidePlan wp = plan_wide(m, n, k, Q38A_EPI_RESIDUAL, cus);
-  if (wp.tiles > 0 && wp.splits > 1) {
-    out[0] = std::max(out[0], size_t(wp.tiles) * wp.splits * wp.nb * 256);
-    out[1] = std::max(out[1], size_t(wp.tiles));
+  // the tile kernel's plan depends on m through its rows of 128-row tiles only
+  for (int r = kSmallMaxRows + 1; r <= m && !big_fits(r, n, cus); r = (r + 127) / 128 * 128 + 1) {
+    const TilePlan t = plan_tile(r, n, k, cus, kTileMaxSplits);
+    need(t.partial_floats(), t.counters());
   }
   return Q38A_OK;
 }
@@ -1894,7 +1886,7 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
     return ap ? launch_qk_norm_rope_append(*ap, *b, *kv, stream) : Q38A_OK;
   };
   // large M: 256 x 256 tiles with the weights dequantised once per workgroup, when those tiles fill
-  // the CUs
+  // the CUs (below that the 128-column tiles, and their K slices, keep more of them busy)
   if (m > kSmallMaxRows && big_fits(m, w.n, cus)) {
     g.tiles_n = w.n / kTileN;
     g.splits = 1;
@@ -1945,6 +1937,9 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
 #undef Q38A_WIDE
     return then_append();
   }
+  // the other launches up to 64 rows: per layer 33 rows 23.2 us (in-projection with the append) and
+  // 20.8 us (o-projection), 64 rows 26.8 and 22.3; the 64 x 256-column split-K tiles took 91.6, 65, 120
+  // and 79 us
   if (!mi) {
     SmallPlan sp = plan_small(m, w.n, w.k, ep.kind, cus);
     if (sp.splits > 1 && (!ws.partials || !ws.counters || ws.partial_floats < sp.partial_floats(m) || ws.num_counters < sp.tiles)) {

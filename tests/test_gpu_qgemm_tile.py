@@ -99,3 +99,29 @@ def test_tile_without_workspace(orc):
     small = gemm.BQWeight(w.desc.lo, None, w.desc.scales, 4, 512, 4096, 512)  # (refused before it is read)
     with pytest.raises(Q38AError):
         gemm.qgemm(a_t.data_ptr(), 64, small, ep, none, stream())
+
+
+@pytest.mark.parametrize("n,k", [(14336, 5120), (5120, 6144), (512, 4096)])
+def test_workspace_serves_fewer_rows(n, k):
+    """The workspace of m rows is enough for every smaller m, also where m itself needs none."""
+    last = (0, 0)
+    for m in [*range(1, 140), *range(140, 2300, 37)]:
+        size = gemm.workspace_size(m, n, k)
+        assert size[0] >= last[0] and size[1] >= last[1], (m, size, last)
+        last = size
+
+
+def test_smaller_launch_in_a_larger_workspace(orc):
+    """128 rows of the in-projection's shape split K; they run in the workspace of 512 rows, which do not."""
+    n, k, m = 14336, 5120, 128
+    w = Weight(orc, 4, n, k, seed=9)
+    a = randn_bf16(np.random.default_rng(8), (m, k))
+    a_t = dev(a)
+    ws, keep = workspace(512, n, k)
+    out = torch.zeros(m * n, dtype=torch.int16, device="cuda")
+    ep = gemm.GemmEpilogue(gemm.EPI_STORE_BF16, out.data_ptr(), n, 0, None, None, None, None, 0, 1e-6)
+    print(f"larger workspace: m={m} n={n} k={k}", flush=True)
+    gemm.qgemm(a_t.data_ptr(), m, w.desc, ep, ws, stream())
+    rows = np.r_[0:2, m - 1:m]
+    close(bf16_bits_to_f32(host(out, np.uint16).reshape(m, n)[rows]), orc.qgemm(a[rows], w.w_exact, 3), "bf16", a[rows],
+          np.abs(w.w_exact))
