@@ -484,6 +484,12 @@ __device__ inline void copy_to_lds(__amdgpu_buffer_rsrc_t r, u32x4* dst, int vof
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voffset, soffset, 0, 0);
 }
 
+// s_waitcnt's immediate for "at most n vector memory loads in flight" (gfx9 encoding, the other counters
+// not waited for). The loads retire in order, so it says that everything issued before the newest n has
+// landed. n counts loads that the code after it reads: the compiler deletes the others, and a wait that
+// counts a deleted load leaves the copy before it in flight.
+constexpr int vm_in_flight(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
+
 // One thread's share of a step's weights: NS 16-k steps of one lane word (their low nibbles, 32
 // bits a step) and the high bits of those steps.
 template <int NS>
@@ -686,8 +692,11 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto step = [&](int t, auto curc) {
+  // TAIL: one of the up to three steps after the unrolled loop; no later step reads what they would load.
+  constexpr int kCopies = 4, kLoads = (BITS == 4 ? 1 : 2) + 2;  // of a step: A copies; words and scales
+  auto step = [&](int t, auto curc, auto tailc) {
     constexpr int cur = decltype(curc)::value;
+    constexpr bool TAIL = decltype(tailc)::value;
     const TileWords<NS>& wnext = wq[(cur + 1) & 3];
     const int wbuf = (cur & 1) ^ 1 ^ ahead;
     bf16x8_t ao[4][2], bo[2][4];
@@ -707,13 +716,14 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
     dma_a(t + 2, abuf == 0 ? 2 : abuf - 1);
     // the wait at the phase's end counts the loads issued after the copies: keep that order
     __builtin_amdgcn_sched_barrier(0);
-    load_words(wq[cur], t + 4 + ahead);
-    load_scales(sc[(cur + 3) & 3], t + 3);
-    __builtin_amdgcn_sched_barrier(0);
-    // the copies of step t + 1 have landed: at most the loads issued after them are in flight (vmcnt
-    // counts in order: per step the words' low nibbles, the high bits of 5- and 6-bit codes, two
-    // scales, and the four copies of step t + 2)
-    __builtin_amdgcn_s_waitcnt(BITS == 4 ? 0x0F7A : 0x0F7C);
+    if constexpr (!TAIL) {
+      load_words(wq[cur], t + 4 + ahead);
+      load_scales(sc[(cur + 3) & 3], t + 3);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the copies of step t + 1 have landed: after them went out that step's loads, the copies of step
+    // t + 2 and this step's loads; in the tail only the newest copies are sure to have
+    __builtin_amdgcn_s_waitcnt(vm_in_flight(TAIL ? kCopies : kLoads + kCopies + kLoads));
     phase_end();
     __builtin_amdgcn_s_setprio(1);
     fold(1, last_sc);  // the previous step's second column block
@@ -748,14 +758,14 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
   if (wave >= 4) phase_end();
   int t = 0;
   for (; t + 3 < steps; t += 4) {
-    step(t, i0{});
-    step(t + 1, i1{});
-    step(t + 2, i2{});
-    step(t + 3, i3{});
+    step(t, i0{}, std::false_type{});
+    step(t + 1, i1{}, std::false_type{});
+    step(t + 2, i2{}, std::false_type{});
+    step(t + 3, i3{}, std::false_type{});
   }
-  if (t < steps) step(t, i0{});
-  if (t + 1 < steps) step(t + 1, i1{});
-  if (t + 2 < steps) step(t + 2, i2{});
+  if (t < steps) step(t, i0{}, std::true_type{});
+  if (t + 1 < steps) step(t + 1, i1{}, std::true_type{});
+  if (t + 2 < steps) step(t + 2, i2{}, std::true_type{});
   if (wave < 4) phase_end();
   fold(1, last_sc);
   // the copies past the last step have landed and every wave is past its last operand read: LDS is
@@ -994,8 +1004,10 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto half = [&](int g, auto curc, auto hc) {
+  constexpr int kCopies = 4, kLoads = (BITS == 4 ? 1 : 2) + 1;  // of a group: A copies; words and scale
+  auto half = [&](int g, auto curc, auto hc, auto tailc) {  // TAIL: as in qgemm_tile_kernel
     constexpr int cur = decltype(curc)::value, H = decltype(hc)::value;
+    constexpr bool TAIL = decltype(tailc)::value;
     bf16x8_t ao[2][2], bo[2][4];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -1012,11 +1024,11 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
     if constexpr (H == 0) {
       dma_a(g + 2, abuf == 0 ? 2 : abuf - 1);
     } else {
-      load_words(cur, g + 4);
-      // the copies of group g + 1 have landed: after them went out one group's words, the copies of
-      // group g + 2 and another group's words (two loads a word for 4-bit codes, else three)
+      if constexpr (!TAIL) load_words(cur, g + 4);
+      // the copies of group g + 1 have landed: after them went out one group's loads, the copies of
+      // group g + 2 and another group's loads; in the tail only the newest copies are sure to have
       __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_waitcnt(BITS == 4 ? 0x0F78 : 0x0F7A);
+      __builtin_amdgcn_s_waitcnt(vm_in_flight(TAIL ? kCopies : kLoads + kCopies + kLoads));
     }
     phase_end();
     __builtin_amdgcn_s_setprio(1);
@@ -1042,20 +1054,20 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
     phase_end();
   };
   if (wave >= 4) phase_end();
-  auto group = [&](int g, auto curc) {
-    half(g, curc, i0{});
-    half(g, curc, i1{});
+  auto group = [&](int g, auto curc, auto tailc) {
+    half(g, curc, i0{}, tailc);
+    half(g, curc, i1{}, tailc);
   };
   int g = 0;
   for (; g + 3 < G; g += 4) {
-    group(g, i0{});
-    group(g + 1, i1{});
-    group(g + 2, i2{});
-    group(g + 3, i3{});
+    group(g, i0{}, std::false_type{});
+    group(g + 1, i1{}, std::false_type{});
+    group(g + 2, i2{}, std::false_type{});
+    group(g + 3, i3{}, std::false_type{});
   }
-  if (g < G) group(g, i0{});
-  if (g + 1 < G) group(g + 1, i1{});
-  if (g + 2 < G) group(g + 2, i2{});
+  if (g < G) group(g, i0{}, std::true_type{});
+  if (g + 1 < G) group(g + 1, i1{}, std::true_type{});
+  if (g + 2 < G) group(g + 2, i2{}, std::true_type{});
   if (wave < 4) phase_end();
   // the copies past the last group have landed and every wave is past its last operand read
   __builtin_amdgcn_s_waitcnt(0);
@@ -1535,8 +1547,7 @@ __global__ void __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per
   auto compute = [&](int d) {
     // this group's copies have landed: at most the next group's loads are in flight
     constexpr int kNext = 4 * RB + 2 * (BITS == 4 ? 2 : 3);
-    static_assert(kNext < 16, "vmcnt's low field");
-    __builtin_amdgcn_s_waitcnt(0x0F70 | kNext);
+    __builtin_amdgcn_s_waitcnt(vm_in_flight(kNext));
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     u32x4 A[RB][4];
