@@ -489,6 +489,8 @@ __device__ inline void copy_to_lds(__amdgpu_buffer_rsrc_t r, u32x4* dst, int vof
 // landed. n counts loads that the code after it reads: the compiler deletes the others, and a wait that
 // counts a deleted load leaves the copy before it in flight.
 constexpr int vm_in_flight(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
+// As well, that every LDS operation of the wave has completed.
+constexpr int vm_in_flight_lds_done(int n) { return vm_in_flight(n) & ~0x0F00; }
 
 // One thread's share of a step's weights: NS 16-k steps of one lane word (their low nibbles, 32
 // bits a step) and the high bits of those steps.
@@ -678,10 +680,12 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
   // One step in two phases with a barrier after each: operand reads and loads, then the MFMAs with the
   // folds and the dequantisation in their shadow. Waves 4-7 run half a step behind waves 0-3, so of a
   // SIMD's two waves one is in each phase. Waves 0-3 dequantise step t + 1 beside the MFMAs of step t,
-  // waves 4-7 step t + 2 (ahead = 1): either is then complete when waves 0-3 start to read it, and
-  // its buffer was last read, by waves 4-7, before the first of them writes to it. The copies of a
-  // step's A rows go out two steps ahead into the buffer read a step ago. cur = t % 4 is a
-  // compile-time constant, so the register rings are indexed statically.
+  // waves 4-7 step t + 2 (ahead = 1): either is then complete when waves 0-3 start to read it. The copies
+  // of a step's A rows go out two steps ahead into the buffer read a step ago. Both overwrite what waves
+  // 4-7 read in the phase before, so a wave's operand reads have returned when it passes the barrier
+  // after them (in-projection, 512 rows: 390 us with the wait; with it only where tiles of 256 rows need
+  // it, 391; o-projection, 519 rows: 253, 256). cur = t % 4 is a compile-time constant, so the register
+  // rings are indexed statically.
   int abuf = 0;  // t mod 3: the A buffer of step t
   // (A plain barrier: __syncthreads would wait for every copy in flight. The empty assembly keeps the
   // compiler from moving memory accesses across it.)
@@ -722,8 +726,9 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
       __builtin_amdgcn_sched_barrier(0);
     }
     // the copies of step t + 1 have landed: after them went out that step's loads, the copies of step
-    // t + 2 and this step's loads; in the tail only the newest copies are sure to have
-    __builtin_amdgcn_s_waitcnt(vm_in_flight(TAIL ? kCopies : kLoads + kCopies + kLoads));
+    // t + 2 and this step's loads; in the tail only the newest copies are sure to have. And the operand
+    // reads have returned.
+    __builtin_amdgcn_s_waitcnt(vm_in_flight_lds_done(TAIL ? kCopies : kLoads + kCopies + kLoads));
     phase_end();
     __builtin_amdgcn_s_setprio(1);
     fold(1, last_sc);  // the previous step's second column block
@@ -875,7 +880,7 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
 // As the tiles above, with eight waves of 64 rows x 128 columns and the weights staged in LDS as
 // bf16(code x scale) (the reference's own weight rounding, qgemm.cu), so that the MFMA accumulates
 // across groups directly. A group goes in two halves of 32 k, each a memory phase (12 operand reads,
-// and the copies of A two groups ahead or the weights' loads) and a compute phase (16 MFMAs with half a
+// in the second half also the copies of A two groups ahead and the weights' loads) and a compute phase (16 MFMAs with half a
 // lane word's dequantisation, ~3 vector instructions per MFMA), waves 4-7 one phase behind. The tile
 // count fills the CUs, so no split-K.
 //
@@ -994,7 +999,10 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
   // waves 4-7 one phase behind waves 0-3. A half's operands are complete when waves 0-3 read them (the
   // codes' same half of the group before was dequantised at least one phase earlier by either set of
   // waves), and the buffers are free when they are written: half H of group g + 1 goes where group
-  // g - 1's half H was, last read by waves 4-7 two phases before. cur = g % 4 is a compile-time constant,
+  // g - 1's half H was, the copies of group g + 2 (in the second half of group g) where group g - 1's rows
+  // were; waves 4-7 read either two phases before at the latest, and used it in the one between. (In the
+  // first half the copies would meet their last reads: 1,201 us with a wait for those, in-projection of
+  // 2,048 rows over four layers, 1,194 so.) cur = g % 4 is a compile-time constant,
   // so the register ring is indexed statically.
   int abuf = 0;  // g mod 3
   auto phase_end = [&]() {  // (as in qgemm_tile_kernel)
@@ -1021,9 +1029,9 @@ __global__ void __launch_bounds__(kBigThreads) __attribute__((amdgpu_waves_per_e
         bo[s][j] = *reinterpret_cast<const bf16x8_t*>(&sh.s.b[cur & 1][4 * wn + j][2 * H + s][lane][0]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (H == 0) {
+    if constexpr (H == 1) {
       dma_a(g + 2, abuf == 0 ? 2 : abuf - 1);
-    } else {
+      __builtin_amdgcn_sched_barrier(0);
       if constexpr (!TAIL) load_words(cur, g + 4);
       // the copies of group g + 1 have landed: after them went out one group's loads, the copies of
       // group g + 2 and another group's loads; in the tail only the newest copies are sure to have

@@ -5,9 +5,11 @@ stay in flight across barriers. A count that includes loads the compiler deleted
 that the next step reads.
 
 The walk keeps, for a wave, the loads in flight in order and how many barriers each copy has passed.
-  * Tile kernels: a copy is read by the other waves two barriers before its own wave reads it, so one in
-    flight at its third barrier (`overdue`; the seventh where a step is two halves) must never be
-    followed by another operand read.
+  * Tile kernels: a copy is read by the other waves one barrier before its own wave reads it, so one in
+    flight at its third barrier (`overdue`; the fifth where a step is two halves) must never be followed
+    by another operand read.
+  * Tile kernels: what a wave reads from LDS is written again by other waves `late` + 1 barriers later at the
+    earliest, so its reads have returned when it arrives at the barrier before that.
   * 9- to 64-row kernel (wave-private buffers): at an operand read only the next group's copies may be in
     flight."""
 import os
@@ -103,7 +105,7 @@ def waited(ins, counter):
 
 
 @pytest.mark.parametrize("name,overdue", [(f"qgemm_tile_kernel {b} {wm}", 2) for b in (4, 5, 6) for wm in (2, 4)] +
-                         [(f"qgemm_big_kernel {b}", 6) for b in (4, 5, 6)])
+                         [(f"qgemm_big_kernel {b}", 4) for b in (4, 5, 6)])
 def test_copies_land_before_they_are_read(kernels, name, overdue):
     late = []
 
@@ -128,6 +130,31 @@ def test_copies_land_before_they_are_read(kernels, name, overdue):
 
     walk(kernels[name], visit, ((), False))
     assert not late, f"{len(late)} paths read A rows whose copy may not have landed"
+
+
+# 128- and 256-row tiles: waves read a buffer in one phase and, in the next, others dequantise or copy into
+# it. 256 x 256 tiles: copies and codes go into what was read at least two phases before.
+@pytest.mark.parametrize("name,late", [(f"qgemm_tile_kernel {b} {wm}", 0) for b in (4, 5, 6) for wm in (2, 4)] +
+                         [(f"qgemm_big_kernel {b}", 1) for b in (4, 5, 6)])
+def test_reads_return_before_their_buffer_is_written(kernels, name, late):
+    bad = []
+
+    def visit(ins, lds):  # the LDS operations in flight, oldest first: -1, or the barriers a read has passed
+        if ins.startswith("ds_"):
+            lds += (0 if ins.startswith("ds_read") else -1,)
+            assert len(lds) < 64
+        n = waited(ins, "lgkmcnt")
+        if n is not None:
+            lds = lds[len(lds) - n:] if n else ()
+        elif ins.startswith("s_barrier"):
+            if any(r >= late for r in lds):
+                bad.append(ins)
+                return None
+            lds = tuple(r + 1 if r >= 0 else r for r in lds)
+        return lds
+
+    walk(kernels[name], visit, ())
+    assert not bad, f"{len(bad)} paths pass a barrier with reads outstanding of a buffer that is written next"
 
 
 @pytest.mark.parametrize("name", [f"qgemm_small_kernel {b} {rb} {cw}" for b in (4, 5, 6) for rb in (1, 2) for cw in (1, 2)])
