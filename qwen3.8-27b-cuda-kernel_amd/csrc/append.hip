@@ -178,9 +178,9 @@ qk_norm_rope_append_rows_kernel(AppendArgs p, BatchArgs batch, KvArgs kv) {
     return;
   }
   // int8: a 64-dim group is four lanes
-  float amax = 0.0f;
+  float amax = fabsf(x[0]);  // (as quantize_row_int8: a group of NaNs alone keeps NaN as its scale)
 #pragma unroll
-  for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(x[e]));
+  for (int e = 1; e < 16; ++e) amax = fmaxf(amax, fabsf(x[e]));
   amax = fmaxf(amax, as_f32(dpp_move<kDppXor1>(as_u32(amax))));
   amax = fmaxf(amax, as_f32(dpp_move<kDppXor2>(as_u32(amax))));
   if (!store_ok) return;

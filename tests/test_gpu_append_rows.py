@@ -58,3 +58,47 @@ def test_rows_kernel_matches_one_row_per_wave(nq, nkv, kv_dtype):
     assert_bits_equal(got[0][0], got[1][0], "q")
     assert_bits_equal(got[0][1], got[1][1], "pool bytes")
     assert (got[0][0].reshape(M, -1)[-30:] == 0x7E00).all()
+
+
+@pytest.mark.parametrize("kv_dtype", [q38a.KV_INT8, q38a.KV_INT8_VT, q38a.KV_BF16])
+def test_non_finite_rows_match_one_row_per_wave(kv_dtype):
+    """NaNs and infinities in q, k and v: the same bytes from both kernels. A K row with a NaN or a V
+    group of NaNs alone keeps NaN as its scale, so that attention over it shows it; a NaN among other
+    values of a V group is quantised to 0."""
+    rng = np.random.default_rng(5)
+    M, nkv = 8192 // 32 + 5, 4
+    b = Batch([(0, 7, M)])
+    bt, pages = paged_layout(rng, [7 + M])
+    x = randn_bf16(rng, (M, LD)).reshape(M, LD // HD, HD)
+    nan, inf = np.uint16(0x7FC1), np.uint16(0x7F80)
+    k, v = 2 * NQ, 2 * NQ + nkv
+    x[3, 5, 17] = nan
+    x[4, 6, 40:44] = inf
+    x[9, k + 1, 200] = nan  # the whole normalised row is NaN
+    x[10, k + 2, 5] = inf
+    x[11, v, 64:128] = nan
+    x[12, v + 1, 70] = nan
+    x[13, v + 2, 130] = inf | np.uint16(0x8000)
+    proj = dev(x.reshape(M, LD))
+    odd = torch.zeros(M * LD + 4, dtype=torch.int16, device="cuda")
+    odd[4:] = proj.view(-1)
+    ones = dev(np.ones(HD, np.float32))
+    rope = rope_dev(7 + M)
+    got = []
+    for p in (proj, odd[4:]):
+        pool = Pool(kv_dtype, pages, bt)
+        q = torch.zeros(M * NQ * HD, dtype=torch.int16, device="cuda")
+        print(f"append non-finite: dtype={kv_dtype}", flush=True)
+        q38a.qk_norm_rope_append(append_params(p, ones, ones, q, rope), b.desc, pool.desc, stream())
+        torch.cuda.synchronize()
+        got.append((host(q, np.uint16), pool.download()))
+    assert_bits_equal(got[0][0], got[1][0], "q")
+    assert_bits_equal(got[0][1], got[1][1], "pool bytes")
+    if kv_dtype == q38a.KV_INT8:
+        page = got[0][1].reshape(pages, -1)
+        at = lambda m: (page[bt[0, (7 + m) // 64]], (7 + m) % 64)
+        scales = lambda m, plane, h: at(m)[0][2 * nkv * 64 * HD:].view(np.uint16).reshape(2, nkv, 64, 4)[plane, h, at(m)[1]]
+        assert (scales(9, 0, 1) == 0x7E00).all()
+        s = scales(11, 1, 0)
+        assert s[1] == 0x7E00 and (s[[0, 2, 3]] < 0x7C00).all()
+        assert (scales(12, 1, 1) < 0x7C00).all()
