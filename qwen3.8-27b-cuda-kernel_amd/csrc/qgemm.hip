@@ -25,6 +25,7 @@
 //     with write-through stores, counts its arrival on a per-tile counter, and the last to arrive sums
 //     the slices in slice order (deterministic) and runs the epilogue, then resets the counter.
 //   * the o-projection's A merged in the loader has a split-K kernel of its own (qgemv_kernel).
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -1511,7 +1512,9 @@ struct alignas(16) SmallShared {
   int last;
 };
 
-template <int BITS, int RB, int CW>
+// DMA: A by copies into LDS, which need rows of 16-byte alignment; otherwise through registers, with
+// loads of any alignment.
+template <int BITS, int RB, int CW, bool DMA>
 __global__ void __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(2))) qgemm_small_kernel(GemmArgs a) {
   constexpr int KW = kSmallWaves / CW, kCols = 64 * CW;
   constexpr int kVals = CW * RB * 2 * 16 * 64 / kSmallThreads;  // outputs per thread
@@ -1539,14 +1542,23 @@ __global__ void __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) C[rb][0] = C[rb][1] = float16_t{};
   BWords B[2][2];
+  u32x4 R[2][DMA ? 1 : 4 * RB];  // without DMA: the groups' A rows on their way to LDS
   // unconditional loads (past the share's end they repeat its last group, cached and unused): a load
   // under a branch would make the loop's waits conservative
   auto load_group = [&](int d, int g) {
     const int gc = g < g1 - 1 ? g : (g1 > g0 ? g1 - 1 : gb);
     __builtin_amdgcn_sched_barrier(0);  // (the buffer's operand reads have returned: their MFMAs are issued)
 #pragma unroll
-    for (int i = 0; i < 4 * RB; ++i)
-      copy_to_lds(ars, &sh.a[wave][d][8 * i][0], (i & 1 ? avoff ^ 64 : avoff) + 16 * i * a.k, 128 * gc);
+    for (int i = 0; i < 4 * RB; ++i) {
+      const int off = (i & 1 ? avoff ^ 64 : avoff) + 16 * i * a.k;
+      if constexpr (DMA) {
+        copy_to_lds(ars, &sh.a[wave][d][8 * i][0], off, 128 * gc);
+      } else {
+        // (rows past M load row 0: an output row depends on its own row only)
+        const int at = 8 * i + (lane >> 3) < a.m ? off : avoff - (lane >> 3) * a.k * 2;
+        __builtin_memcpy(&R[d][i], reinterpret_cast<const char*>(a.a) + at + 128 * gc, 16);
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < 2; ++j) load_bwords<BITS, kNonTemporal>(B[d][j], bp, nb0 + j, gc, G, lane);
@@ -1555,7 +1567,12 @@ __global__ void __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per
   auto compute = [&](int d) {
     // this group's copies have landed: at most the next group's loads are in flight
     constexpr int kNext = 4 * RB + 2 * (BITS == 4 ? 2 : 3);
-    __builtin_amdgcn_s_waitcnt(vm_in_flight(kNext));
+    if constexpr (DMA) {
+      __builtin_amdgcn_s_waitcnt(vm_in_flight(kNext));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4 * RB; ++i) sh.a[wave][d][8 * i + (lane >> 3)][lane & 7] = R[d][i];
+    }
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     u32x4 A[RB][4];
@@ -1835,14 +1852,35 @@ void launch_gemv(bool ev1, dim3 grid, hipStream_t stream, const GemmArgs& g, con
 }
 
 template <int BITS>
-void launch_small(int m, int cw, dim3 grid, hipStream_t stream, const GemmArgs& g) {
+void launch_small(int cw, dim3 grid, hipStream_t stream, const GemmArgs& g) {
   const dim3 block(kSmallThreads);
-  if (m > 32) {
-    if (cw == 1) hipLaunchKernelGGL((qgemm_small_kernel<BITS, 2, 1>), grid, block, 0, stream, g);
-    else hipLaunchKernelGGL((qgemm_small_kernel<BITS, 2, 2>), grid, block, 0, stream, g);
+  if (g.m > 32) {
+    if (cw == 1) hipLaunchKernelGGL((qgemm_small_kernel<BITS, 2, 1, true>), grid, block, 0, stream, g);
+    else hipLaunchKernelGGL((qgemm_small_kernel<BITS, 2, 2, true>), grid, block, 0, stream, g);
   } else {
-    if (cw == 1) hipLaunchKernelGGL((qgemm_small_kernel<BITS, 1, 1>), grid, block, 0, stream, g);
-    else hipLaunchKernelGGL((qgemm_small_kernel<BITS, 1, 2>), grid, block, 0, stream, g);
+    if (cw == 1) hipLaunchKernelGGL((qgemm_small_kernel<BITS, 1, 1, true>), grid, block, 0, stream, g);
+    else hipLaunchKernelGGL((qgemm_small_kernel<BITS, 1, 2, true>), grid, block, 0, stream, g);
+  }
+}
+
+// A without 16-byte alignment: any number of rows, kSmallMaxRows a launch, on 128-column tiles.
+template <int BITS>
+void launch_unaligned(const SmallPlan& sp, hipStream_t stream, GemmArgs g) {
+  const dim3 grid(unsigned(sp.tiles), unsigned(sp.splits)), block(kSmallThreads);
+  const size_t rows = g.m;
+  for (size_t done = 0; done < rows; done += kSmallMaxRows) {
+    g.m = int(std::min(rows - done, size_t(kSmallMaxRows)));
+    if (g.m > 32) hipLaunchKernelGGL((qgemm_small_kernel<BITS, 2, 2, false>), grid, block, 0, stream, g);
+    else hipLaunchKernelGGL((qgemm_small_kernel<BITS, 1, 2, false>), grid, block, 0, stream, g);
+    g.a += size_t(kSmallMaxRows) * g.k;
+    if (g.kind == Q38A_EPI_RESIDUAL) {
+      g.residual += size_t(kSmallMaxRows) * g.n;
+      g.xbf += size_t(kSmallMaxRows) * g.n;
+      g.partials_out += size_t(kSmallMaxRows) * g.norm_blocks;
+    } else {
+      g.out = static_cast<char*>(g.out) + size_t(kSmallMaxRows) * g.ldo * (g.kind == Q38A_EPI_STORE_F32 ? 4 : 2);
+      if (g.partials_in) g.partials_in += size_t(kSmallMaxRows) * g.norm_blocks;
+    }
   }
 }
 
@@ -1918,7 +1956,11 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
     }
     return then_append();
   }
-  if (m > kSmallMaxRows) {
+  // The kernels below copy A to LDS 16 bytes at a time, which is only sure to be right for aligned
+  // rows; other A goes through registers, 64 rows a launch (in-projection, four layers: 16 rows 111 us
+  // against 69, 64 rows 174 against 107, 512 rows 1,300 against 380).
+  const bool copy_a = aligned(A, 16);
+  if (m > kSmallMaxRows && copy_a) {
     TilePlan tp = plan_tile(m, w.n, w.k, cus, kTileMaxSplits);
     if (!tp.fits(ws)) {
       if (tile_needs_workspace(m, w.n, w.k, cus)) return set_error(Q38A_ERR_INVALID, small_ws);
@@ -1960,16 +2002,25 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
   // 20.8 us (o-projection), 64 rows 26.8 and 22.3; the 64 x 256-column split-K tiles took 91.6, 65, 120
   // and 79 us
   if (!mi) {
-    SmallPlan sp = plan_small(m, w.n, w.k, ep.kind, cus);
+    SmallPlan sp = plan_small(m, w.n, w.k, copy_a ? ep.kind : int(Q38A_EPI_RESIDUAL), cus);  // (128-column tiles)
     if (sp.splits > 1 && (!ws.partials || !ws.counters || ws.partial_floats < sp.partial_floats(m) || ws.num_counters < sp.tiles)) {
       if (pl.tiles_n == 0 && tile_needs_workspace(m, w.n, w.k, cus)) return set_error(Q38A_ERR_INVALID, small_ws);
       sp.splits = 1;
     }
+    if (!copy_a) {
+      switch (w.bits) {
+        case 4: launch_unaligned<4>(sp, stream, g); break;
+        case 5: launch_unaligned<5>(sp, stream, g); break;
+        case 6: launch_unaligned<6>(sp, stream, g); break;
+        default: return set_error(Q38A_ERR_UNSUPPORTED, "qgemm: %d-bit weights are not supported", w.bits);
+      }
+      return then_append();
+    }
     const dim3 sgrid(unsigned(sp.tiles), unsigned(sp.splits));
     switch (w.bits) {
-      case 4: launch_small<4>(m, sp.cw, sgrid, stream, g); break;
-      case 5: launch_small<5>(m, sp.cw, sgrid, stream, g); break;
-      case 6: launch_small<6>(m, sp.cw, sgrid, stream, g); break;
+      case 4: launch_small<4>(sp.cw, sgrid, stream, g); break;
+      case 5: launch_small<5>(sp.cw, sgrid, stream, g); break;
+      case 6: launch_small<6>(sp.cw, sgrid, stream, g); break;
       default: return set_error(Q38A_ERR_UNSUPPORTED, "qgemm: %d-bit weights are not supported", w.bits);
     }
     return then_append();

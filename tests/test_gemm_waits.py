@@ -56,11 +56,11 @@ def kernels(tmp_path_factory):
             m = re.match(r"[0-9a-f]+ <(\S+)>:", line)
             if m:
                 k = re.search(r"(qgemm_(?:tile|big|small)_kernel)I(\w*?)EEv", m[1])
-                code = out.setdefault(k[1] + " " + " ".join(re.findall(r"Li(\d+)E", k[2] + "E")), []) if k else None
+                code = out.setdefault(k[1] + " " + " ".join(re.findall(r"L[ib](\d+)E", k[2] + "E")), []) if k else None
             elif code is not None and "//" in line:
                 ins, rest = line.split("//", 1)
                 code.append((int(rest.split(":")[0], 16), ins.strip()))
-    assert len(out) == 6 + 3 + 12, sorted(out)
+    assert len(out) == 6 + 3 + 18, sorted(out)
     return out
 
 
@@ -157,7 +157,7 @@ def test_reads_return_before_their_buffer_is_written(kernels, name, late):
     assert not bad, f"{len(bad)} paths pass a barrier with reads outstanding of a buffer that is written next"
 
 
-@pytest.mark.parametrize("name", [f"qgemm_small_kernel {b} {rb} {cw}" for b in (4, 5, 6) for rb in (1, 2) for cw in (1, 2)])
+@pytest.mark.parametrize("name", [f"qgemm_small_kernel {b} {rb} {cw} 1" for b in (4, 5, 6) for rb in (1, 2) for cw in (1, 2)])
 def test_wave_private_copies_land_before_they_are_read(kernels, name):
     copies = 4 * int(name.split()[2])  # of a group
     late = []

@@ -56,3 +56,38 @@ def test_small_rows(orc, bits, m, n, k):
         gemm.qgemm(a_t.data_ptr(), m, w.desc, ep, ws, stream())
         check_residual(orc, w, a, res0, host(res).reshape(m, n), host(xbf, np.uint16).reshape(m, n),
                        host(pout).reshape(m, n // 128))
+
+
+@pytest.mark.parametrize("m,n,k,kind", [(5, 256, 576, gemm.EPI_STORE_BF16), (9, 512, 320, gemm.EPI_STORE_F32),
+                                        (33, 12288, 128, gemm.EPI_STORE_BF16), (64, 2560, 1088, gemm.EPI_RESIDUAL),
+                                        (129, 512, 640, gemm.EPI_RESIDUAL), (200, 256, 448, gemm.EPI_STORE_BF16)])
+def test_unaligned_a(orc, m, n, k, kind):
+    """A on a 2-byte boundary, which the copies into LDS are not made for: rows through registers, 64 a
+    launch. The same bits as the oracle's bounds allow, with every row's scale, residual and sums in place."""
+    w = Weight(orc, 6, n, k, seed=m + 1)
+    rng = np.random.default_rng(m + k)
+    a = randn_bf16(rng, (m, k))
+    shifted = torch.zeros(m * k + 8, dtype=torch.int16, device="cuda")
+    shifted[3:3 + m * k] = dev(a).view(-1)
+    ap = shifted.data_ptr() + 6
+    hidden = 128 * max(1, k // 128)
+    partials = rng.uniform(50.0, 200.0, (m, hidden // 128)).astype(np.float32)
+    p_t = dev(partials)
+    ws, keep = workspace(m, n, k)
+    print(f"unaligned A: m={m} n={n} k={k} kind={kind}", flush=True)
+    if kind == gemm.EPI_RESIDUAL:
+        res0 = rng.standard_normal((m, n)).astype(np.float32)
+        res, xbf = dev(res0), torch.zeros(m * n, dtype=torch.int16, device="cuda")
+        pout = torch.zeros(m * (n // 128), dtype=torch.float32, device="cuda")
+        ep = gemm.GemmEpilogue(kind, None, 0, 0, res.data_ptr(), xbf.data_ptr(), pout.data_ptr(), None, 0, 1e-6)
+        gemm.qgemm(ap, m, w.desc, ep, ws, stream())
+        check_residual(orc, w, a, res0, host(res).reshape(m, n), host(xbf, np.uint16).reshape(m, n),
+                       host(pout).reshape(m, n // 128))
+        return
+    f32 = kind == gemm.EPI_STORE_F32
+    out = torch.zeros(m * n, dtype=torch.float32 if f32 else torch.int16, device="cuda")
+    ep = gemm.GemmEpilogue(kind, out.data_ptr(), n, 0, None, None, None, p_t.data_ptr(), hidden, 1e-6)
+    gemm.qgemm(ap, m, w.desc, ep, ws, stream())
+    got = host(out).reshape(m, n) if f32 else bf16_bits_to_f32(host(out, np.uint16).reshape(m, n))
+    want = orc.qgemm(a, w.w_exact, 3, partials_in=partials, hidden=hidden)
+    close(got, want, "unaligned", a, w.w_offset_mag, row_scales(partials, hidden), out="f32" if f32 else "bf16")
