@@ -14,7 +14,7 @@ from util import assert_bits_equal, bf16_bits_to_f32, randn_bf16
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(9, 256, 64), (31, 512, 320), (32, 12288, 128), (33, 12288, 192), (64, 2560, 1088), (63, 256, 2048),
-          (5, 256, 576)]
+          (5, 256, 576), (33, 256, 64), (64, 256, 192)]
 
 
 @pytest.mark.parametrize("bits", [4, 5, 6])
