@@ -7,7 +7,18 @@ kernels' orders and requires: where the test admits the tree's sum, its rounded 
 left-to-right one's, bit for bit; a mean on a rounding boundary is not admitted; and N(0,1) rows are."""
 import numpy as np
 
-from test_append_exact_sum import bf16_round, tree_sum
+from util import bf16_bits_to_f32, f32_to_bf16_bits
+
+
+def tree_sum(x):
+    """One row per wave: 4 values per lane in order, then the cross-lane steps (lane ^ 1, lane ^ 2, the mirrors
+    within 8 and 16 lanes, lane ^ 16, lane ^ 32)."""
+    part = [sum(float(x[4 * l + e]) ** 2 for e in range(4)) for l in range(64)]
+    for p in (lambda l: l ^ 1, lambda l: l ^ 2, lambda l: (l & ~7) | (7 - (l & 7)), lambda l: (l & ~15) | (15 - (l & 15)),
+              lambda l: l ^ 16, lambda l: l ^ 32):
+        part = [part[l] + part[p(l)] for l in range(64)]
+    assert len(set(part)) == 1
+    return part[0]
 
 
 def sum16(x):
@@ -50,7 +61,7 @@ def test_mean_criterion():
             x = boundary_row(rng)
         else:
             x = rng.normal(0, 1, 256) * np.exp2(rng.integers(-40, 6, 256) * (rng.random(256) < 0.1))
-        x = bf16_round(x).astype(np.float64)
+        x = bf16_bits_to_f32(f32_to_bf16_bits(x.astype(np.float32))).astype(np.float64)
         seq = 0.0
         for v in x:
             seq = seq + v * v

@@ -1,7 +1,7 @@
 """GPU parity of the projection GEMMs (include/q38a_gemm.h) against the oracle: q38a_qgemm with its
 StoreBF16 (folded-norm row scale), StoreF32 and Residual epilogues on BQ4/5/6 weights written in the
 reference's file layout and repacked by the library (reference src/kernels/qgemm.cu:285-384), and
-the in-projection with the fused norm / RoPE / append, which must equal q38a_qgemm followed by
+the in-projection with the norm / RoPE / append in the same call, which must equal q38a_qgemm followed by
 q38a_qk_norm_rope_append bit for bit (q, K/V bytes and scales, the gate columns of proj).
 
 The oracle's double-precision product is taken over the weights the kernel path multiplies by:
