@@ -43,7 +43,8 @@ qk_norm_rope_append_kernel(AppendArgs p, BatchArgs batch, KvArgs kv, int jobs) {
   // q head r at column r*256; k head h at (2nq + h)*256; v head h at (2nq + nkv + h)*256
   const int col = (L.r < p.nq ? L.r : p.nq + L.r) * kHeadDim;
   L.pos = batch.tok_pos[L.m];
-  L.raw = *reinterpret_cast<const uint2*>(p.proj + size_t(L.m) * p.ld_proj + col + 4 * lane);
+  // (any alignment: the in-projection call takes every row stride and 2-byte aligned rows)
+  __builtin_memcpy(&L.raw, p.proj + size_t(L.m) * p.ld_proj + col + 4 * lane, sizeof(L.raw));
   row_meta(p, batch, kv, lane, L);
   append_row(p, kv, stage[wave], lane, L);
 }

@@ -7,9 +7,11 @@ import pytest
 import torch
 
 import q38a
+from q38a import gemm
 from gpu_util import HD, LD, NQ, Batch, Pool, append_params, dev, host, paged_layout, rope_dev, stream
 from test_append_mean import boundary_row
 from test_gpu_append import run_append
+from test_gpu_qgemm import InProj, workspace
 from util import assert_bits_equal, f32_to_bf16_bits, randn_bf16
 
 pytestmark = pytest.mark.gpu
@@ -102,3 +104,28 @@ def test_non_finite_rows_match_one_row_per_wave(kv_dtype):
         s = scales(11, 1, 0)
         assert s[1] == 0x7E00 and (s[[0, 2, 3]] < 0x7C00).all()
         assert (scales(12, 1, 1) < 0x7C00).all()
+
+
+@pytest.mark.parametrize("M", [5, 40, 257])
+def test_in_projection_any_row_stride(orc, M):
+    """The in-projection with its append, proj's rows of an odd stride and on a 2-byte boundary (the append
+    reads them back): the gate columns, q and the pool as with aligned rows, bit for bit."""
+    ip = InProj(orc, [(60, M)], seed=M)
+
+    def run(ld, shift):
+        pool = Pool(ip.kv_dtype, ip.pages, ip.bt, fill=ip.pool_host)
+        proj = torch.zeros(M * ld + shift, dtype=torch.int16, device="cuda")[shift:]
+        q = torch.zeros(M * NQ * HD, dtype=torch.int16, device="cuda")
+        ws, keep = workspace(M, ip.n, ip.k)
+        ep = gemm.GemmEpilogue(gemm.EPI_STORE_BF16, proj.data_ptr(), ld, 0, None, None, None, ip.p_t.data_ptr(), ip.k,
+                               1e-6)
+        print(f"in-projection: M={M} ld={ld} shift={shift}", flush=True)
+        gemm.qgemm_qkv_append(ip.a_t.data_ptr(), M, ip.w.desc, ep, ws,
+                              append_params(proj, ip.qn_t, ip.kn_t, q, ip.rope_t, ld=ld), ip.b.desc, pool.desc, stream())
+        torch.cuda.synchronize()
+        return host(proj, np.uint16).reshape(M, ld)[:, NQ * HD:2 * NQ * HD], host(q, np.uint16), pool.download()
+
+    want = run(LD, 0)
+    for ld, shift in ((LD + 1, 0), (LD + 2, 0), (LD, 3)):
+        for got, ref, what in zip(run(ld, shift), want, ("gate", "q fp16", "pool bytes")):
+            assert_bits_equal(got, ref, what)
