@@ -129,47 +129,82 @@ __device__ inline int decode_pages(const BatchArgs& batch, int s) {
 
 // Pages per item of a decode launch: every row needs at most max_splits items per kv head, and the
 // batch yields about target_items items. FIT (a grid of one workgroup per target item, each taking
-// every target-th item): not more than target_items, so that no workgroup has a second item while the
-// others are done. Each row's last item is partly filled, so whole pages of psum * nkv / target_items
-// alone overshoot the target about every sixth batch (8 rows, 203K tokens on bf16 pages: 520 items
-// of 25 pages against 512, the step 190 us; 504 items of 26 pages, 160 us).
+// every target-th item): longer items, not more than target_items of them, so that no workgroup has a
+// second item while the others are done. Each row's last item is partly filled, so whole pages of
+// psum * nkv / target_items alone overshoot the target about every sixth batch (8 rows, 203K tokens on
+// bf16 pages: 520 items of 25 pages against 512, the step 190 us; 504 items of 26 pages, 160 us).
+//
+// Not where the longest item would grow by more than half, half the overshoot's share and a page: few
+// workgroups with a second item then cost less than all with a longer one, or too few with one (rows of equal
+// length go from three items each to two, from two to one). The step in us, rows x tokens, int8 pages, first
+// choice and longer items:
+//   43 x 1,900: 516 of 11 pages 53.8, 344 of 15 52.5    43 x 4,700: 516 of 25 103.5, 344 of 37 100.7
+//   45 x 1,076: 540 of  6 pages 39.5, 360 of  9 39.8    33 x 6,000: 528 of 25 104.0, 396 of 32  90.9
+//   65 x   400: 520 of  4 pages 35.6, 260 of  7 35.7    80 x 1,000: 640 of 10  57.8, 320 of 16  57.5
+//   90 x 2,000: 720 of 23 pages 103.8, 360 of 32 95.0
+// and past the bound:
+//   75 x 2,000: 600 of 19 pages 87.9, 300 of 32 90.8    66 x 1,000: 528 of 9 52.1, 264 of 16 55.3
+//   66 x 3,000: 528 of 25 pages 107, 264 of 47 121
 template <bool FIT>
 __device__ inline DecodePlan wave_decode_plan(const BatchArgs& batch, int nkv, int max_splits, int target_items) {
   const int lane = threadIdx.x & 63;
   DecodePlan pl;
   pl.pages0 = decode_pages(batch, lane);
-  int psum = pl.pages0, pmax = pl.pages0;  // pages: < 2^31 for any pool a 32-bit block table addresses
-  for (int s0 = 64; s0 < batch.num_seqs; s0 += 64) {
+  constexpr int kHeld = FIT ? 128 : 64;  // rows whose pages stay in registers until the plan is made
+  const int pages1 = FIT && batch.num_seqs > 64 ? decode_pages(batch, 64 + lane) : 0;
+  int psum = pl.pages0 + pages1, pmax = max(pl.pages0, pages1);  // (< 2^31 for any pool a block table addresses)
+  for (int s0 = kHeld; s0 < batch.num_seqs; s0 += 64) {
     const int p = decode_pages(batch, s0 + lane);
     psum += p;
     pmax = max(pmax, p);
   }
   psum = __builtin_amdgcn_readfirstlane(wave_sum_i(psum));  // (scalars: cp must stay wave-uniform)
-  pmax = wave_max_i(pmax);
+  pmax = __builtin_amdgcn_readfirstlane(wave_max_i(pmax));
   const int by_splits = ceil_div_i(pmax, max_splits);
   const int by_target = int((static_cast<long long>(psum) * nkv + target_items - 1) / target_items);
   pl.cp = __builtin_amdgcn_readfirstlane(max(1, max(by_splits, by_target)));
-  auto count = [&]() {
-    int items = ceil_div_i(pl.pages0, pl.cp);
-    for (int s0 = 64; s0 < batch.num_seqs; s0 += 64) items += ceil_div_i(decode_pages(batch, s0 + lane), pl.cp);
-    return __builtin_amdgcn_readfirstlane(wave_sum_i(items) * nkv);
-  };
   if constexpr (FIT) {
-    // (Counting costs a wave reduction on the way to the first loads: not where a partly filled item
-    // per row cannot reach the target. One item per row and head too many: nothing to be gained.)
-    const long long most = static_cast<long long>(psum) + static_cast<long long>(batch.num_seqs) * pl.cp;
-    if (pl.cp > 1 && most * nkv > static_cast<long long>(target_items) * pl.cp && batch.num_seqs * nkv <= target_items) {
-      // longer items in steps of the overshoot's share
-      int items = count();
-      for (int i = 0; i < 8 && items > target_items; ++i) {
-        pl.cp += max(1, int(static_cast<long long>(pl.cp) * (items - target_items) / target_items));
-        items = count();
+    // (Counting is on the way to the first loads: not where a partly filled item per row cannot reach the
+    // target. One item per row and head too many: nothing to be gained.)
+    const int first = pl.cp, rows = batch.num_seqs;
+    const long long most = static_cast<long long>(psum) + static_cast<long long>(rows) * first;
+    if (first > 1 && first < 1024 && rows <= kHeld && rows * nkv <= target_items &&
+        most * nkv > static_cast<long long>(target_items) * first) {
+      // Items beyond the target with c pages each: ceil(p / c) = floor(p / c + (c - 1/2) / c), whose argument is
+      // 1/2c (2^-12) from an integer at least and off by less (p / c <= target / nkv), without a division per
+      // row. (Each count is ~0.2 us of the decode and of the merge launch: two after the first, no more.)
+      const float p0 = float(pl.pages0), p1 = float(pages1);
+      auto count = [&](int c) {
+        const float inv = __builtin_amdgcn_rcpf(float(c)), up = (float(c) - 0.5f) * inv;
+        int n = int(__builtin_floorf(__builtin_fmaf(p0, inv, up)));
+        if (rows > 64) n += int(__builtin_floorf(__builtin_fmaf(p1, inv, up)));
+        return __builtin_amdgcn_readfirstlane(wave_sum_i(n) * nkv) - target_items;
+      };
+      const int over = count(first);
+      if (over > 0) {
+        // rows of about one length: as many items each as the target takes; else so much longer as brings the
+        // items that are not the rows' last, half filled ones down by the overshoot, once more if that was not
+        // enough (98 of 100 batches fit then, 92 at once)
+        // (in 32 bits: psum <= target first / nkv, and 64-bit divisions cost a microsecond here)
+        auto up_div = [](int a, int b) { return int((uint32_t(a) + uint32_t(b) - 1u) / uint32_t(b)); };
+        int left = over, c = first;
+        const bool even = 10 * psum >= 9 * rows * pmax;
+        for (int i = 0; i < 2 && left > 0; ++i) {
+          c = even && i == 0 ? max(first + 1, up_div(pmax, int(uint32_t(target_items) / uint32_t(rows * nkv))))
+                             : c + up_div(c * left, target_items - rows * nkv / 2);
+          // (left > 0: the first choice stays)
+          if ((min(c, pmax) - first - 1) * 2 * target_items > first * (target_items + over)) break;
+          left = count(c);
+        }
+        if (left <= 0) pl.cp = c;
       }
       pl.cp = __builtin_amdgcn_readfirstlane(pl.cp);
     }
     pl.items = 0;  // (not used: the kernels stride over the items until wave_locate finds none)
   } else {
-    pl.items = count();
+    int items = ceil_div_i(pl.pages0, pl.cp);
+    for (int s0 = 64; s0 < batch.num_seqs; s0 += 64) items += ceil_div_i(decode_pages(batch, s0 + lane), pl.cp);
+    pl.items = __builtin_amdgcn_readfirstlane(wave_sum_i(items) * nkv);
   }
   return pl;
 }
