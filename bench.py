@@ -219,17 +219,18 @@ INPROJ_COPIES = 8  # 8 x 48 MB of weights: more than the 256 MB MALL, as 16 laye
 
 def inproj_setup(name):
     """The attention layer's in-projection (W [q | gate | k | v] = 14,336 x 5,120, bq5 as the reference
-    model stores it, reference docs/FORMAT.md 1.3) on the decode batch of config 2 (M = 8) or the
-    prefill chunk of config 3 (M = 2,048). Launch i uses weight copy i % INPROJ_COPIES, so weights
-    stream from HBM as a step's different layers do. Returns (gemm(i), gemm + append(i), fused(i),
-    facts)."""
+    model stores it, reference docs/FORMAT.md 1.3) on the decode batch of config 2 (in_proj_b8: M = 8) or
+    a chunk of M tokens (in_proj_M; the prefill chunk of config 3: 2,048). Launch i uses weight copy
+    i % INPROJ_COPIES, so weights stream from HBM as a step's different layers do. Returns (gemm(i),
+    gemm + append(i), the same in one call(i), facts)."""
     import torch
     import q38a
     from q38a import gemm
     from q38a.workloads import LD, DecodeBatch, RaggedBatch, decode_contexts
     s = torch.cuda.current_stream().cuda_stream
     gen = torch.Generator(device="cuda").manual_seed(0)
-    b = DecodeBatch(decode_contexts("decode_b8"), seed=0) if name.endswith("b8") else RaggedBatch([(6000, 2048)], seed=0)
+    rows = name.split("_")[-1]
+    b = DecodeBatch(decode_contexts("decode_b8"), seed=0) if rows == "b8" else RaggedBatch([(6000, int(rows))], seed=0)
     m = b.batch.num_tokens
     K, bits = 5120, 5
     ws_ = [random_bq_weight(LD, K, bits, gen) for _ in range(INPROJ_COPIES)]
@@ -254,8 +255,8 @@ def inproj_setup(name):
 
 
 def inproj_config(name, steps, warmup):
-    """The in-projection (inproj_setup) timed three ways: the GEMM alone, GEMM + append (two
-    launches, proj written and re-read), and the fused launch (q38a_qgemm_qkv_append)."""
+    """The in-projection (inproj_setup) timed three ways: the GEMM alone, GEMM and append as two calls,
+    and as one (q38a_qgemm_qkv_append; "fused_ms")."""
     import torch
     run_gemm, run_unfused, run_fused, f = inproj_setup(name)
 
@@ -451,8 +452,8 @@ def profile_workload(name, reps=20):
         ap, kvd = rb.attention_params(), rb.kv_desc(0)
         q38a.qk_norm_rope_append(rb.append_params(), rb.batch, kvd, s)
         run = lambda i: q38a.attention_ragged(ap, rb.batch, kvd, s)  # noqa: E731
-    elif base in ("in_proj_b8", "in_proj_2048"):
-        run, _, _, keep = inproj_setup(base)
+    elif base in ("in_proj_b8", "in_proj_32", "in_proj_200", "in_proj_512", "in_proj_2048"):
+        _, _, run, keep = inproj_setup(base)
     elif base in ("o_proj_b8", "o_proj_b8_fused"):
         unfused, fused, _, keep = oproj_setup("o_proj_b8")
         run = fused if base.endswith("fused") else unfused
@@ -569,6 +570,36 @@ def mfma_summary(d, out=None, simds=1024):
     print(text)
     if out:
         open(out, "w").write(text + "\n")
+
+
+def units_summary(d, cus=256):
+    """What the units of the chip do under each kernel, from a rocprofv3 --pmc run of
+    SQ_VALU_MFMA_BUSY_CYCLES, SQ_ACTIVE_INST_VALU, SQ_LDS_IDX_ACTIVE, SQ_LDS_BANK_CONFLICT, SQ_INSTS_VALU,
+    SQ_INSTS_MFMA and GRBM_GUI_ACTIVE over `bench.py --profile`. MFMA busy: relative to the MFMA probe
+    kernel's. VALU and LDS busy: SQ_ACTIVE_INST_VALU and SQ_LDS_IDX_ACTIVE per CU and GPU-active cycle
+    (rocprofv3's VALUBusy and LdsUtil expressions; GRBM_GUI_ACTIVE here is a sum over the 8 XCDs).
+    Bank conflicts: their share of the LDS-active cycles. Clock: GPU-active cycles of an XCD over the
+    dispatch's duration (under ~20 us too short to mean anything)."""
+    import collections
+    per = collections.defaultdict(lambda: collections.defaultdict(float))
+    calls = collections.defaultdict(dict)
+    for r in _csv_rows(d, "counter_collection.csv"):
+        k = short_name(r["Kernel_Name"])
+        if k.startswith("q38a::"):
+            per[k][r["Counter_Name"]] += float(r["Counter_Value"])
+            calls[k][r["Dispatch_Id"]] = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
+    raw = {k: c["SQ_VALU_MFMA_BUSY_CYCLES"] / c["GRBM_GUI_ACTIVE"] for k, c in per.items()}
+    probe = max(raw.values())
+    print("| kernel | dispatches | average us | clock GHz | MFMA busy / probe | VALU busy | LDS busy | bank conflicts | "
+          "VALU instructions per MFMA |")
+    print("|---|---|---|---|---|---|---|---|---|")
+    for k, c in sorted(per.items()):
+        cycles = c["GRBM_GUI_ACTIVE"] / 8 * cus
+        lds, mfma = c["SQ_LDS_IDX_ACTIVE"], c["SQ_INSTS_MFMA"]
+        us = sum(calls[k].values())
+        print(f"| {k} | {len(calls[k])} | {us / len(calls[k]):.1f} | {c['GRBM_GUI_ACTIVE'] / 8 / us / 1e3:.2f} | "
+              f"{raw[k] / probe:.3f} | {c['SQ_ACTIVE_INST_VALU'] / cycles:.3f} | {lds / cycles:.3f} | {c['SQ_LDS_BANK_CONFLICT'] / lds if lds else 0:.3f} | "
+              f"{(c['SQ_INSTS_VALU'] - mfma) / mfma if mfma else float('nan'):.1f} |")
 
 
 def short_name(n):
@@ -748,9 +779,12 @@ def main():
     ap.add_argument("--pmc-out", default=None)
     ap.add_argument("--stats-summary", metavar="DIR")
     ap.add_argument("--mfma-summary", metavar="DIR")
+    ap.add_argument("--units-summary", metavar="DIR")
     args = ap.parse_args()
     if args.mfma_summary:
         return mfma_summary(args.mfma_summary, out=args.pmc_out)
+    if args.units_summary:
+        return units_summary(args.units_summary)
     if args.pmc_summary:
         return pmc_summary(*args.pmc_summary, out=args.pmc_out)
     if args.stats_summary:
