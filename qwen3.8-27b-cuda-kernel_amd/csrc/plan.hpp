@@ -150,11 +150,11 @@ __device__ inline DecodePlan wave_decode_plan(const BatchArgs& batch, int nkv, i
   const int lane = threadIdx.x & 63;
   DecodePlan pl;
   pl.pages0 = decode_pages(batch, lane);
-  constexpr int kHeld = FIT ? 128 : 64;  // rows whose pages stay in registers until the plan is made
-  const int pages1 = FIT && batch.num_seqs > 64 ? decode_pages(batch, 64 + lane) : 0;
-  int psum = pl.pages0 + pages1, pmax = max(pl.pages0, pages1);  // (< 2^31 for any pool a block table addresses)
-  for (int s0 = kHeld; s0 < batch.num_seqs; s0 += 64) {
+  int psum = pl.pages0, pmax = pl.pages0;  // pages: < 2^31 for any pool a 32-bit block table addresses
+  int pages1 = 0;                          // of rows 64..127, where they are counted again
+  for (int s0 = 64; s0 < batch.num_seqs; s0 += 64) {
     const int p = decode_pages(batch, s0 + lane);
+    if (FIT && s0 == 64) pages1 = p;
     psum += p;
     pmax = max(pmax, p);
   }
@@ -168,7 +168,7 @@ __device__ inline DecodePlan wave_decode_plan(const BatchArgs& batch, int nkv, i
     // target. One item per row and head too many: nothing to be gained.)
     const int first = pl.cp, rows = batch.num_seqs;
     const long long most = static_cast<long long>(psum) + static_cast<long long>(rows) * first;
-    if (first > 1 && first < 1024 && rows <= kHeld && rows * nkv <= target_items &&
+    if (first > 1 && first < 1024 && rows <= 128 && rows * nkv <= target_items &&
         most * nkv > static_cast<long long>(target_items) * first) {
       // Items beyond the target with c pages each: ceil(p / c) = floor(p / c + (c - 1/2) / c), whose argument is
       // 1/2c (2^-12) from an integer at least and off by less (p / c <= target / nkv), without a division per
