@@ -1,9 +1,10 @@
 /*
  * q38a GEMMs on either side of the attention path: the in-projection that produces `proj`, with
  * the q/k RMSNorm + RoPE + KV append optionally in the same call, and the o-projection that consumes
- * the attention output, with the decode split merge optionally fused into its A loader. Weights are the reference's BQ format (docs/FORMAT.md section 2: b-bit codes in 64-wide
- * groups along K with one bf16 scale per (row, group)), repacked once at load time into this
- * library's MFMA layout (q38a_bq_repack). Same conventions as q38a.h: device pointers, asynchronous
+ * the attention output, with the decode split merge optionally fused into its A loader. Weights are
+ * the reference's BQ format (docs/FORMAT.md section 2: b-bit codes in 64-wide groups along K with one
+ * bf16 scale per (row, group)), repacked once at load time into this library's MFMA layout
+ * (q38a_bq_repack). Same conventions as q38a.h: device pointers, asynchronous
  * on `stream`, no allocation, int status + q38a_last_error().
  */
 #ifndef Q38A_GEMM_H
@@ -85,8 +86,9 @@ int q38a_qgemm(const uint16_t* a, int m, const q38a_bq_weight* w, const q38a_gem
  * weight (nq + nq + 2 nkv heads of 256 rows), ep a STORE_BF16 epilogue whose out is proj. Runs the GEMM
  * into proj and then the append launch on it: the same bits as q38a_qgemm followed by
  * q38a_qk_norm_rope_append (append->proj and ld_proj must describe ep->out). Callers may rely on the
- * gate columns of proj, which attention reads, q_out and the cache; the q, k and v columns of proj are
- * unspecified. No counterpart in the reference (the producer side of the attention path). */
+ * gate columns of proj, which attention reads, q_out and the cache. The q, k and v columns of proj are
+ * written at every m, with values that callers may not rely on (builds that ran the append in the GEMM's
+ * epilogue left them alone for small m). No counterpart in the reference (the producer side of the attention path). */
 int q38a_qgemm_qkv_append(const uint16_t* a, int m, const q38a_bq_weight* w, const q38a_gemm_epilogue* ep,
                           const q38a_gemm_workspace* ws, const q38a_qk_norm_rope_params* append,
                           const q38a_batch_desc* batch, const q38a_kv_cache_desc* kv, void* stream);

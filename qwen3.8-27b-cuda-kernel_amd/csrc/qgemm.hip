@@ -445,7 +445,8 @@ __device__ inline void store_block(const GemmArgs& a, const OutBlock& ot, int ro
 // zero) and C += scale * T in fp32 when the group is done: the codes are exact, so the only
 // roundings are the fp32 sums'. One column block's T is folded while the other block's MFMAs run,
 // and the last one's beside the next step's first MFMAs. KP: 64-k groups per step. With 256 rows a step
-// is one group; with 128 rows two sets of four waves take one group each, and the sets' sums are added through LDS at the end (set 0 + set 1).
+// is one group; with 128 rows two sets of four waves take one group each, and the sets' sums are added
+// through LDS at the end (set 0 + set 1).
 //
 // Bound: the VALU beside the MFMA. Per 64 x 64 x 64 wave step 16 MFMAs (512 cycles) against 64 folds
 // and 50 (5-bit codes, 256 rows) or 100 dequantisation instructions; two waves per SIMD hide about six
@@ -886,7 +887,8 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
 // count fills the CUs, so no split-K.
 //
 // Bound: MFMA, at the clock the card holds under it. In-projection at 2,048 rows (448 tiles on 256 CUs: 2
-// rounds for 1.75): 301 -> 265 us against the form with all waves in step and 2-byte stores (1,136 TFLOP/s; hipBLASLt's plain bf16 product 245-256 us).
+// rounds for 1.75): 301 -> 265 us against the form with all waves in step and 2-byte stores (1,136 TFLOP/s;
+// hipBLASLt's plain bf16 product 245-256 us on the same card; 285 and 327 us on cards with lower clocks).
 constexpr int kBigRows = 256;
 constexpr int kBigWaves = 8;
 constexpr int kBigThreads = 64 * kBigWaves;
@@ -1487,9 +1489,10 @@ __global__ void __launch_bounds__(64 * kWideWaves) qgemv_wide_kernel(GemmArgs a)
 // streams its weights from HBM into registers (every weight is dequantised once, by the wave whose
 // columns it is, so they are not staged) and copies its A rows, which all workgroups share, from the
 // L2 into an LDS buffer of its own, both one group ahead. (A rows loaded straight into the operand
-// layout touched four times the cache lines: 24 instead of 20.7 us at 32 rows, 34 at 64.) Codes as bf16 128 + u; the group's products start from -(128 + 2^(b-1)) times the rows'
-// sums (four more MFMAs of A against a constant, shared by the two column blocks), so T is A . codes
-// and a group costs one fma per output. The K parts' sums meet in LDS in part order; with a K split over
+// layout touched four times the cache lines: 24 instead of 20.7 us at 32 rows, 34 at 64.) Codes as bf16
+// 128 + u; the group's products start from -(128 + 2^(b-1)) times the rows' sums (four more MFMAs of A
+// against a constant, shared by the two column blocks), so T is A . codes and a group costs one fma per
+// output. The K parts' sums meet in LDS in part order; with a K split over
 // workgroups (CW = 2) the last to arrive adds the slices in slice order.
 //
 // Bound: the weight stream and, around it, one round trip of first loads and the sums' way through
@@ -1784,7 +1787,8 @@ struct TilePlan {
 // The height and slice count of the least estimated time, in us, from a sweep over both on the in-
 // and the o-projection at 48 to 2,048 rows: rounds of one workgroup per CU, each of steps of 0.9 us
 // (256 rows) or 1.12 us (128 rows, two groups), 12 us around them (first loads, epilogue) and, split,
-// 5 + 3 s us for the hand-off. Within 6% of the best measured choice at every size of the sweep;
+// 5 + 3 s us for the hand-off. Within 6% of the best measured choice at every size of the sweep; on seven
+// other weights (n 1,024 to 34,816, k 2,048 to 17,408, 96 to 1,000 rows) within 3% at 27 of 38 sizes, 20% at worst;
 // e.g. in-projection: 128 rows 2 slices of 128-row tiles 38 us (1: 53, 4: 53), 384 rows 256-row
 // tiles 83 us (128-row tiles 109); o-projection: 256 rows 3 slices of 128-row tiles 43 us (1: 72).
 TilePlan plan_tile(int m, int n, int k, int cus, int max_splits) {
@@ -1807,8 +1811,9 @@ TilePlan plan_tile(int m, int n, int k, int cus, int max_splits) {
   return best;
 }
 
-// Launches of fewer than two 64 x 256 tiles a CU are refused without the planned split workspace;
-// larger ones run unsplit without it (they fill the CUs anyway).
+// Without the planned split workspace, launches of fewer than two 64 x 256 tiles a CU are refused, whatever
+// tiles they take; larger ones run unsplit (they fill the CUs anyway). What callers may leave out thus stays
+// the same from one choice of kernels to the next.
 bool tile_needs_workspace(int m, int n, int k, int cus) {
   return ((m + 63) / 64) * (n / kTileN) < 2 * cus && k / 64 >= 8;
 }
@@ -1900,6 +1905,8 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
   if (m <= 0) return Q38A_OK;
   int cus = 0;
   if (int rc = device_cu_count(&cus)) return rc;
+  // (Up to 32 rows every call has to meet the limits of the split-K kernel, which only the merged A takes
+  // now: what was refused stays refused.)
   const GemvPlan pl = plan_gemv(m, w.n, w.k, cus);
   const char* small_ws = "qgemm: workspace too small (q38a_qgemm_workspace_size)";
   if (pl.tiles_n > 0) {

@@ -1,5 +1,5 @@
 """ctypes binding of the projection GEMMs (include/q38a_gemm.h): BQ weight repacking, q38a_qgemm
-(reference kernels.h:120 qgemm) and the in-projection with the fused append."""
+(reference kernels.h:120 qgemm) and the in-projection with the append in the same call."""
 import ctypes
 
 import numpy as np

@@ -61,7 +61,8 @@ def fitted_plan(pages, target, max_splits):
     (45, 3000, 0, True), (43, 1900, 0, True), (33, 6000, 0, True), (80, 1000, 0, True), (90, 2000, 0, True),
     (110, 1800, 0, True), (65, 400, 0, True), (126, 1500, 0, False), (128, 129, 0, False),
     (140, 500, 0, False), (8, 15000, 12000, None), (21, 4000, 700, None), (53, 2200, 1800, None),
-    (100, 900, 800, None), (1, 130000, 0, False), (4, 16000, 12000, True), (20, 9000, 6000, True), (65, 700, 600, True), (86, 1500, 1200, True), (107, 1500, 1200, None)])
+    (100, 900, 800, None), (1, 130000, 0, False), (4, 16000, 12000, True), (20, 9000, 6000, True),
+    (65, 700, 600, True), (86, 1500, 1200, True), (107, 1500, 1200, None)])
 def test_item_lengths(rows, tokens, spread, longer):
     """Keys of zeros give every position the weight 1, so an item's sum of weights is its tokens."""
     target, splits = 2 * torch.cuda.get_device_properties(0).multi_processor_count, 64
