@@ -1949,9 +1949,13 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
     if (int rc = check_hip(hipGetLastError(), "qgemm launch")) return rc;
     return ap ? launch_qk_norm_rope_append(*ap, *b, *kv, stream) : Q38A_OK;
   };
+  // The tile, large-M and 9- to 64-row kernels copy A to LDS 16 bytes at a time, which is only sure to be right
+  // for aligned rows; other A goes through registers, 64 rows a launch (in-projection, four layers: 16 rows
+  // 111 us against 69, 64 rows 174 against 107, 512 rows 1,300 against 380).
+  const bool copy_a = aligned(A, 16);
   // large M: 256 x 256 tiles with the weights dequantised once per workgroup, when those tiles fill
   // the CUs (below that the 128-column tiles, and their K slices, keep more of them busy)
-  if (m > kSmallMaxRows && big_fits(m, w.n, cus)) {
+  if (m > kSmallMaxRows && copy_a && big_fits(m, w.n, cus)) {
     g.tiles_n = w.n / kTileN;
     g.splits = 1;
     const dim3 bgrid(unsigned(((m + kBigRows - 1) / kBigRows) * g.tiles_n)), bblock{unsigned(kBigThreads)};
@@ -1963,10 +1967,6 @@ int launch_qgemm(const uint16_t* A, int m, const q38a_bq_weight& w, const q38a_g
     }
     return then_append();
   }
-  // The kernels below copy A to LDS 16 bytes at a time, which is only sure to be right for aligned
-  // rows; other A goes through registers, 64 rows a launch (in-projection, four layers: 16 rows 111 us
-  // against 69, 64 rows 174 against 107, 512 rows 1,300 against 380).
-  const bool copy_a = aligned(A, 16);
   if (m > kSmallMaxRows && copy_a) {
     TilePlan tp = plan_tile(m, w.n, w.k, cus, kTileMaxSplits);
     if (!tp.fits(ws)) {

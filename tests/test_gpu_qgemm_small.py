@@ -60,7 +60,8 @@ def test_small_rows(orc, bits, m, n, k):
 
 @pytest.mark.parametrize("m,n,k,kind", [(5, 256, 576, gemm.EPI_STORE_BF16), (9, 512, 320, gemm.EPI_STORE_F32),
                                         (33, 12288, 128, gemm.EPI_STORE_BF16), (64, 2560, 1088, gemm.EPI_RESIDUAL),
-                                        (129, 512, 640, gemm.EPI_RESIDUAL), (200, 256, 448, gemm.EPI_STORE_BF16)])
+                                        (129, 512, 640, gemm.EPI_RESIDUAL), (200, 256, 448, gemm.EPI_STORE_BF16),
+                                        (1800, 8192, 128, gemm.EPI_STORE_BF16)])
 def test_unaligned_a(orc, m, n, k, kind):
     """A on a 2-byte boundary, which the copies into LDS are not made for: rows through registers, 64 a
     launch. The same bits as the oracle's bounds allow, with every row's scale, residual and sums in place."""
